@@ -24,6 +24,9 @@ SOURCES = [
     "chs_tune.hip",
     "chs_lineop.hip",
     "chs_lineop_x.hip",
+    "chs_rhs.hip",
+    "chs_rhs_x.hip",
+    "chs_rhs_yz.hip",
     "chs_poisson.hip",
     "chs_flow.hip",
     "chs_api.hip",

@@ -47,6 +47,8 @@ Handle::~Handle() {
   poisson.reset();
   plans64.clear();
   plans32.clear();
+  fuse64.clear();
+  fuse32.clear();
   if (stream) (void)hipStreamDestroy(stream);
 }
 
@@ -87,6 +89,36 @@ std::string Handle::plan(int dir, int op, int iacc, const int ibc[2], bool has_f
   mp[key] = std::move(dp);
   return "";
 }
+template <typename T>
+static std::map<PlanKey, std::unique_ptr<DevFusePlan<T>>>& fuse_map(Handle* h);
+template <>
+std::map<PlanKey, std::unique_ptr<DevFusePlan<double>>>& fuse_map<double>(Handle* h) { return h->fuse64; }
+template <>
+std::map<PlanKey, std::unique_ptr<DevFusePlan<float>>>& fuse_map<float>(Handle* h) { return h->fuse32; }
+
+template <typename T>
+std::string Handle::fuse_plan(int dir, int op, const int ibc[2], bool has_fbc, int n_in, int n_out, bool short_form,
+                              const DevFusePlan<T>** out) {
+  PlanKey key{dir, op, desc.iacc, ibc[0], ibc[1], (has_fbc ? 1 : 0) + (short_form ? 2 : 0), n_in, n_out};
+  auto& mp = fuse_map<T>(this);
+  auto it = mp.find(key);
+  if (it == mp.end()) {
+    std::unique_ptr<DevFusePlan<T>> dp(new DevFusePlan<T>());
+    int P = 0, ell = 0, rows = 0;
+    if (fuse_chunks(dir, n_out, short_form, &P, &ell, &rows)) {
+      LinePlan lp;
+      std::string e = make_line_plan(mesh.line_geom(dir), Op(op), desc.iacc, ibc, has_fbc, n_in, n_out, &lp, ell, P);
+      if (!e.empty()) return e;
+      e = upload_fuse_plan<T>(lp, rows, dp.get());
+      if (!e.empty()) return e;
+    }
+    it = mp.emplace(key, std::move(dp)).first;
+  }
+  *out = it->second.get();
+  return "";
+}
+template std::string Handle::fuse_plan<double>(int, int, const int[2], bool, int, int, bool, const DevFusePlan<double>**);
+template std::string Handle::fuse_plan<float>(int, int, const int[2], bool, int, int, bool, const DevFusePlan<float>**);
 template std::string Handle::plan<double>(int, int, int, const int[2], bool, int, int, const DevPlan<double>**);
 template std::string Handle::plan<float>(int, int, int, const int[2], bool, int, int, const DevPlan<float>**);
 

@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <initializer_list>
 #include <string>
 #include <vector>
 
@@ -54,6 +55,19 @@ struct RhsWork {
   T* scratch_side[2] = {nullptr, nullptr};  // the same for operators on the side streams
   long scratch_n = 0;
   bool ready = false;
+};
+
+// Fused plans of the constant-property sub-step: x and z (periodic) and, with
+// y walls, the y operators by their boundary kinds.
+template <typename T>
+struct FusedPlans {
+  const DevFusePlan<T>*xi_n, *xd_n, *xi_c, *xd_c;  // interpolation / derivative to nodes, to cells
+  const DevFusePlan<T>*zi_n, *zd_n, *zi_c, *zd_c;
+  const DevFusePlan<T>*yi_n, *yd_n;  // u and w to nodes (wall values)
+  const DevFusePlan<T>*yi_c, *yd_c;  // v to cells
+  const DevFusePlan<T>*ys_c;         // shear flux to cells
+  const DevFusePlan<T>*yf_n;         // normal flux to nodes (wall flux)
+  const DevFusePlan<T>*yp_n;         // pressure to nodes
 };
 
 // The energy right-hand side's operands in the precision T its operators
@@ -194,6 +208,19 @@ class Flow {
                       const T* fbc_cov, const T* fbc_tau, const Field<T>& ca, const Field<T>& cb,
                       const Field<T>& ta, T ts, const Field<T>* tb, T tc, int lane = 0);
   template <typename T> std::string momentum_rhs_t(RhsWork<T>& w, int isub, bool fuse);
+  // the same on the fused operators (constant properties; chs_rhs.h)
+  template <typename T> std::string momentum_fused_t(RhsWork<T>& w, int isub, bool fuse);
+  template <typename T> std::string fused_plans(FusedPlans<T>& f, bool* ok);
+  template <typename T>
+  std::string fused_run(int dir, int kind, const DevFusePlan<T>& dp, std::initializer_list<RhsJob<T>> jobs, int lane = 0);
+  std::string fused_ready(bool* ok);  // every operator of the sub-step has its fused plan (decided once)
+  std::string divergence_fused(double* d);
+  std::string correct(double sc);  // p += phi and the velocity correction
+  std::string correct_fused(double sc);
+  FusedPlans<double> f64;
+  FusedPlans<float> f32;
+  int fused_state = 0;        // 0 not decided, 1 fused, 2 single operators
+  bool bulk_pending = false;  // qx holds q + rhs; the forcing's bulk is subtracted by the x correction
   template <typename T> std::string thermo_first_level(RhsWork<T>& w);
   template <typename T> std::string alloc_thermo_work(RhsWork<T>& w);
   std::string refresh_props();

@@ -927,6 +927,277 @@ std::string Flow::momentum_rhs_t(RhsWork<T>& w, int isub, bool fuse) {
   return "";
 }
 
+// ---------------------------------------------------------------------------
+// The sub-step on the fused operators (chs_rhs.h)
+// ---------------------------------------------------------------------------
+// Grids of up to this many cells take the short chunks.
+constexpr long kShortCells = 1L << 19;
+
+template <typename T>
+std::string Flow::fused_plans(FusedPlans<T>& f, bool* ok) {
+  const int(*B)[5][2] = ibc;
+  bool all = true;
+  const bool small = (long)nx * ny * nz <= kShortCells;
+  auto get = [&](const DevFusePlan<T>** p, int dir, int opk, const int* bc, bool fbc, int n_in, int n_out) {
+    std::string e = H->fuse_plan<T>(dir, opk, bc, fbc, n_in, n_out, small, p);
+    if (e.empty() && !(*p)->ok) all = false;
+    return e;
+  };
+  SCHK(get(&f.xi_n, 0, MIDP_C2P, B[0][VV], false, nx, px)); SCHK(get(&f.xd_n, 0, D1_C2P, B[0][VV], false, nx, px));
+  SCHK(get(&f.xi_c, 0, MIDP_P2C, B[0][VU], false, px, nx)); SCHK(get(&f.xd_c, 0, D1_P2C, B[0][VU], false, px, nx));
+  SCHK(get(&f.zi_n, 2, MIDP_C2P, B[2][VU], false, nz, pz)); SCHK(get(&f.zd_n, 2, D1_C2P, B[2][VU], false, nz, pz));
+  SCHK(get(&f.zi_c, 2, MIDP_P2C, B[2][VW], false, pz, nz)); SCHK(get(&f.zd_c, 2, D1_P2C, B[2][VW], false, pz, nz));
+  SCHK(get(&f.yi_n, 1, MIDP_C2P, B[1][VU], wall_y, ny, py)); SCHK(get(&f.yd_n, 1, D1_C2P, B[1][VU], wall_y, ny, py));
+  SCHK(get(&f.yi_c, 1, MIDP_P2C, B[1][VV], wall_y, py, ny)); SCHK(get(&f.yd_c, 1, D1_P2C, B[1][VV], false, py, ny));
+  SCHK(get(&f.ys_c, 1, D1_P2C, mcov[0][1], false, py, ny));
+  SCHK(get(&f.yf_n, 1, D1_C2P, mcov[1][1], wall_y, ny, py));
+  SCHK(get(&f.yp_n, 1, D1_C2P, B[1][VP], wall_y, ny, py));
+  *ok = all;
+  return "";
+}
+
+std::string Flow::fused_ready(bool* ok) {
+  if (fused_state == 0) {
+    // convective and viscous terms of a direction share one operator only
+    // where their boundary kinds agree, and the plans above stand for every
+    // component where the components' kinds do
+    bool same = px == nx && pz == nz;
+    auto eq = [&](const int a[2], const int b[2]) { same = same && a[0] == b[0] && a[1] == b[1]; };
+    for (int c = 0; c < 3; ++c)
+      for (int d = 0; d < 3; ++d) eq(mcov[c][d], mtau[c][d]);
+    eq(mcov[0][1], mcov[2][1]);
+    eq(ibc[1][VU], ibc[1][VW]);
+    for (int d : {0, 2})
+      for (int c = 0; c < 3; ++c) {
+        same = same && mcov[c][d][0] == BC_PERIODIC && mcov[c][d][1] == BC_PERIODIC;
+        for (int v : {VU, VV, VW, VP}) same = same && ibc[d][v][0] == BC_PERIODIC && ibc[d][v][1] == BC_PERIODIC;
+      }
+    bool p64 = false, p32 = true;
+    if (same) {
+      SCHK(fused_plans<double>(f64, &p64));
+      if (p64 && mixed) SCHK(fused_plans<float>(f32, &p32));
+    }
+    fused_state = same && p64 && p32 ? 1 : 2;
+  }
+  *ok = fused_state == 1 && !thermo;
+  return "";
+}
+
+// Line geometry of a job along dir on input A and outputs of extents eo.
+template <typename T>
+static RhsJob<T> fused_job(int dir, const Field<T>& A, const Ext3& eo, const DevFusePlan<T>& p1,
+                           const DevFusePlan<T>* p2 = nullptr) {
+  RhsJob<T> j{};
+  const int* a = A.e.n;
+  j.A = A.p;
+  j.p1 = p1.k;
+  if (p2) j.p2 = p2->k;
+  if (dir == 0) {
+    j.nlines = a[1] * a[2];
+    j.e1 = 1;
+  } else if (dir == 1) {
+    j.nlines = a[0] * a[2];
+    j.e1 = a[0];
+    j.is = a[0]; j.ips = (long)a[0] * a[1];
+    j.os = eo.n[0]; j.ops = (long)eo.n[0] * eo.n[1];
+  } else {
+    j.nlines = a[0] * a[1];
+    j.e1 = a[0];
+    j.is = (long)a[0] * a[1]; j.ips = a[0];
+    j.os = (long)eo.n[0] * eo.n[1]; j.ops = eo.n[0];
+  }
+  return j;
+}
+
+// Grids of up to this many cells put jobs of one kind into one launch.
+constexpr long kGroupCells = 1L << 20;
+
+template <typename T>
+std::string Flow::fused_run(int dir, int kind, const DevFusePlan<T>& dp, std::initializer_list<RhsJob<T>> jobs, int lane) {
+  const hipStream_t s = lane_stream(lane);
+  const bool group = (long)nx * ny * nz <= kGroupCells && H->prof_class < 0;
+  RhsGroup<T> g;
+  auto flush = [&]() -> std::string {
+    if (!g.n) return "";
+    hipEvent_t e0 = nullptr, e1 = nullptr;
+    const bool timed = (H->prof_class == dir) && H->prof_pair(&e0, &e1);
+    if (timed) {
+      (void)hipEventRecord(e0, s);
+      for (int j = 0; j < g.n; ++j) {
+        // fields read and written in T (the second field, the epilogue's), and in FP64
+        const RhsJob<T>& J = g.job[j];
+        const double ni = (double)J.nlines * J.p1.n_in, no = (double)J.nlines * J.p1.n_out;
+        const double rd[6] = {0, 0, 2, 4, 3, 0}, wr[6] = {1, 2, 1, 3, 1, 0};
+        H->prof_bytes += sizeof(T) * (ni * (kind == RK_FINAL ? 2 : 1) + no * (rd[kind] + wr[kind]));
+        if (kind == RK_FINAL) H->prof_bytes += J.q ? 16.0 * no : sizeof(T) * no;
+        if (kind == RK_FINAL && J.tz == T(0)) H->prof_bytes -= sizeof(T) * no;
+        if (kind == RK_CORRECT) H->prof_bytes += 32.0 * no + (J.out32 ? 4.0 * no : 0.0) + (J.add32 ? 4.0 * no : 0.0);
+      }
+    }
+    std::string e = dir == 0 ? launch_rhs_x<T>(kind, dp.rows, g, s) : launch_rhs_yz<T>(kind, dp.rows, g, s);
+    if (timed) (void)hipEventRecord(e1, s);
+    g.n = 0;
+    return e;
+  };
+  for (const RhsJob<T>& j : jobs) {
+    g.job[g.n++] = j;
+    if (!group || g.n == kGroupJobs) SCHK(flush());
+  }
+  return flush();
+}
+
+// Compute_momentum_rhs, the fractional step and the forcing on the fused
+// operators: the same terms as momentum_rhs_t (whose comments give the
+// reference's lines), with the elementwise work in the operators' epilogues.
+// With fuse the state of every component is updated in place (x of a forced
+// flow without its bulk correction, which the x correction applies: a constant
+// has no divergence); without, rhs is left in w.acc[c][0].
+template <typename T>
+std::string Flow::momentum_fused_t(RhsWork<T>& w, int isub, bool fuse) {
+  FusedPlans<T>* fp;
+  if constexpr (sizeof(T) == 8) fp = &f64;
+  else fp = &f32;
+  const FusedPlans<T>& f = *fp;
+  const hipStream_t s = H->stream;
+  const T r = T(rre);
+  const T* fu = wall_y ? w.fby_u : nullptr;
+  const T* fv = wall_y ? w.fby_v : nullptr;
+  const T* fw = wall_y ? w.fby_w : nullptr;
+  auto pair = [&](int dir, const Field<T>& A, const DevFusePlan<T>* pi, const T* fi, const DevFusePlan<T>* pd,
+                  const T* fd, Field<T>& oi, Field<T>& od) {
+    RhsJob<T> j = fused_job<T>(dir, A, oi.e, *pi, pd);
+    j.fbc = fi; j.fbc2 = fd;
+    j.out = oi.p; j.out2 = od.p;
+    return j;
+  };
+  auto shear = [&](int dir, const Field<T>& A, const DevFusePlan<T>* pi, const DevFusePlan<T>* pd, const T* fb,
+                   const Field<T>& oi, const Field<T>& od, Field<T>& out) {
+    RhsJob<T> j = fused_job<T>(dir, A, out.e, *pi, pd);
+    j.fbc = j.fbc2 = fb;
+    j.o1 = oi.p; j.o2 = od.p;
+    j.out = out.p;
+    j.r = r;
+    return j;
+  };
+  auto single = [&](int dir, const Field<T>& A, const DevFusePlan<T>* p, Field<T>& out) {
+    RhsJob<T> j = fused_job<T>(dir, A, out.e, *p);
+    j.out = out.p;
+    return j;
+  };
+  Field<T>*X = w.acc[0], *Y = w.acc[1], *Z = w.acc[2];
+  auto xp_u = pair(0, w.qx, f.xi_c, nullptr, f.xd_c, nullptr, w.qxix, w.qxdx);
+  auto xp_v = pair(0, w.qy, f.xi_n, nullptr, f.xd_n, nullptr, w.qyix, w.qydx);
+  auto xp_w = pair(0, w.qz, f.xi_n, nullptr, f.xd_n, nullptr, w.qzix, w.qzdx);
+  auto yp_v = pair(1, w.qy, f.yi_c, fv, f.yd_c, nullptr, w.qyiy, w.qydy);
+  auto yp_w = pair(1, w.qz, f.yi_n, fw, f.yd_n, fw, w.qziy, w.qzdy);
+  // shear fluxes f_xy, f_xz, f_yz (in qxiy, qxiz, qyiz)
+  auto s_xy = shear(1, w.qx, f.yi_n, f.yd_n, fu, w.qyix, w.qydx, w.qxiy);
+  auto s_xz = shear(2, w.qx, f.zi_n, f.zd_n, nullptr, w.qzix, w.qzdx, w.qxiz);
+  auto s_yz = shear(2, w.qy, f.zi_n, f.zd_n, nullptr, w.qziy, w.qzdy, w.qyiz);
+  // normal fluxes f_zz (qziz), f_xx and f_yy (over qxix, qyiy)
+  RhsJob<T> dv = fused_job<T>(2, w.qz, w.qziz.e, *f.zi_c, f.zd_c);
+  dv.o1 = w.qxdx.p; dv.o2 = w.qydy.p; dv.o3 = w.qxix.p; dv.o4 = w.qyiy.p;
+  dv.out = w.qziz.p;
+  dv.r = r;
+  auto y_x = single(1, w.qxiy, f.ys_c, X[1]);
+  auto x_y = single(0, w.qxiy, f.xd_c, Y[0]);
+  auto z_x = single(2, w.qxiz, f.zd_c, X[2]);
+  auto x_z = single(0, w.qxiz, f.xd_c, Z[0]);
+  auto z_y = single(2, w.qyiz, f.zd_c, Y[2]);
+  auto y_z = single(1, w.qyiz, f.ys_c, Z[1]);
+  // a small grid runs level by level (few, grouped launches); a large one
+  // follows each flux from its making to its two uses while it is in cache
+  SCHK(fused_run<T>(0, RK_PAIR, *f.xi_c, {xp_v, xp_u, xp_w}));
+  SCHK(fused_run<T>(1, RK_SHEAR, *f.yi_n, {s_xy}));
+  SCHK(fused_run<T>(1, RK_PAIR, *f.yi_n, {yp_w}));
+  SCHK(fused_run<T>(1, RK_PAIR, *f.yi_c, {yp_v}));
+  SCHK(fused_run<T>(2, RK_SHEAR, *f.zi_n, {s_xz, s_yz}));
+  if (wall_y) {
+    const DevPlan<T>* P = nullptr;
+    SCHK(H->plan<T>(1, D1_C2P, H->desc.iacc, ibc[1][VV], true, ny, py, &P));
+    SCHK(launch_wall_flux<T>(*P, w.qyiy.e, w.qyiy.p, w.fby_v, r, w.fby_visc, s));
+  }
+  SCHK(fused_run<T>(2, RK_DIV, *f.zi_c, {dv}));
+  SCHK(fused_run<T>(0, RK_SINGLE, *f.xd_c, {x_y, x_z}));
+  SCHK(fused_run<T>(1, RK_SINGLE, *f.ys_c, {y_x, y_z}));
+  SCHK(fused_run<T>(2, RK_SINGLE, *f.zd_c, {z_x, z_y}));
+  // each component's own direction, the pressure gradient and the fractional step
+  const bool forced = H->desc.idriven == 1;
+  const Mesh& m = H->mesh;
+  Field<T>* r0[3] = {&w.mx0, &w.my0, &w.mz0};
+  const Field<double>* qs[3] = {&qx, &qy, &qz};
+  const Field<T>* fl[3] = {&w.qxix, &w.qyiy, &w.qziz};
+  const DevFusePlan<T>* pf[3] = {f.xd_n, f.yf_n, f.zd_n};
+  const DevFusePlan<T>* pp[3] = {f.xd_n, f.yp_n, f.zd_n};
+  for (int c = 0; c < 3; ++c) {
+    RhsJob<T> j = fused_job<T>(c, *fl[c], w.acc[c][0].e, *pf[c], pp[c]);
+    j.A2 = w.pr.p;
+    if (c == 1 && wall_y) {
+      j.fbc = w.fby_visc;
+      j.fbc2 = w.fby_p;
+    }
+    j.o1 = w.acc[c][c == 0 ? 1 : 0].p;
+    j.o2 = w.acc[c][c == 2 ? 1 : 2].p;
+    j.out = w.acc[c][0].p;
+    j.tg = T(tg[isub]); j.tz = T(tz[isub]); j.ta = T(ta[isub]); j.dt = T(dt);
+    j.r0 = r0[c]->p;
+    j.q = fuse ? qs[c]->p : nullptr;
+    if (c == 1 && wall_y && fuse) j.fbw = w64.fby_v;
+    if (c == 0 && forced) {
+      j.partial = partial;
+      j.dyw = dyw_dev;
+      j.dxdz = m.h[0] * m.h[2];
+      j.n2 = ny;
+      if (rhs_x_blocks<T>(j) > npartial) return "fused: too many partial sums";
+    }
+    SCHK(fused_run<T>(c, RK_FINAL, *pf[c], {j}));
+    if (c == 0 && forced)
+      hipLaunchKernelGGL(k_finish_sum, dim3(1), dim3(1024), 0, s, partial, rhs_x_blocks<T>(j), vol, bulk);
+  }
+  bulk_pending = fuse && forced;
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return std::string("momentum_fused: ") + hipGetErrorString(e);
+  return "";
+}
+
+// Divergence of the state on the fused operators.
+std::string Flow::divergence_fused(double* d) {
+  Field<double> D{d, Ext3{{nx, ny, nz}}};
+  RhsJob<double> jx = fused_job<double>(0, qx, D.e, *f64.xd_c), jy = fused_job<double>(1, qy, D.e, *f64.yd_c),
+                 jz = fused_job<double>(2, qz, D.e, *f64.zd_c);
+  jx.out = jy.out = jz.out = d;
+  jy.sOut = jz.sOut = 1.0;
+  SCHK(fused_run<double>(0, RK_SINGLE, *f64.xd_c, {jx}));
+  SCHK(fused_run<double>(1, RK_CORRECT, *f64.yd_c, {jy}));
+  return fused_run<double>(2, RK_CORRECT, *f64.zd_c, {jz});
+}
+
+// Correct_massflux on the fused operators, one lane per component: x also does
+// p += phi (the increment passes that kernel anyway) and the forcing's bulk
+// correction of qx, y sets the wall values (enforce_velo_from_fbc).
+std::string Flow::correct_fused(double sc) {
+  RhsJob<double> jx = fused_job<double>(0, pcor, qx.e, *f64.xd_n), jy = fused_job<double>(1, pcor, qy.e, *f64.yp_n),
+                 jz = fused_job<double>(2, pcor, qz.e, *f64.zd_n);
+  jx.sOut = jy.sOut = jz.sOut = -sc;
+  jx.out = qx.p; jy.out = qy.p; jz.out = qz.p;
+  if (mixed) {
+    jx.out32 = w32.qx.p; jy.out32 = w32.qy.p; jz.out32 = w32.qz.p;
+    jx.add32 = w32.pr.p;
+  }
+  jx.bulk = bulk_pending ? bulk : nullptr;
+  bulk_pending = false;
+  jx.add = pr.p;
+  if (wall_y) {
+    jy.fbc = w64.fby_p;
+    jy.fbw = w64.fby_v;
+  }
+  SCHK(fork());
+  SCHK(fused_run<double>(0, RK_CORRECT, *f64.xd_n, {jx}, 0));
+  SCHK(fused_run<double>(1, RK_CORRECT, *f64.yp_n, {jy}, 1));
+  SCHK(fused_run<double>(2, RK_CORRECT, *f64.zd_n, {jz}, 2));
+  return join();
+}
+
 std::string Flow::refresh_q32() {
   if (!mixed) return "";
   hipStream_t s = H->stream;
@@ -942,7 +1213,9 @@ std::string Flow::refresh_q32() {
 
 std::string Flow::momentum_rhs(int isub, bool fuse) {
   set_lanes();
-  if (!mixed) return momentum_rhs_t<double>(w64, isub, fuse);
+  bool fused = false;
+  SCHK(fused_ready(&fused));
+  if (!mixed) return fused ? momentum_fused_t<double>(w64, isub, fuse) : momentum_rhs_t<double>(w64, isub, fuse);
   // rounded copies of the state for the FP32 right-hand side, unless the
   // last sub-step left them
   if (!q32_fresh) SCHK(refresh_q32());
@@ -957,12 +1230,15 @@ std::string Flow::momentum_rhs(int isub, bool fuse) {
                            pr2.second->p, pr2.second->size());
     g32_fresh = false;
   }
-  const std::string r = momentum_rhs_t<float>(w32, isub, fuse);
+  const std::string r = fused ? momentum_fused_t<float>(w32, isub, fuse) : momentum_rhs_t<float>(w32, isub, fuse);
   if (fuse) q32_fresh = false;  // the state was updated
   return r;
 }
 
 std::string Flow::divergence(double* d) {
+  bool fused = false;
+  SCHK(fused_ready(&fused));
+  if (fused) return divergence_fused(d);
   // of q, or of g = rho u with variable properties (src/eq_continuity.f90:114-117)
   Field<double> D{d, Ext3{{nx, ny, nz}}};
   const Field<double>& ux = thermo ? w64.gx : qx;
@@ -972,6 +1248,28 @@ std::string Flow::divergence(double* d) {
   SCHK(op<double>(w64, 1, D1_P2C, ibc[1][VV], uy, D, nullptr, 1.0, nullptr, 1.0, nullptr, 1.0, 1));
   SCHK(op<double>(w64, 2, D1_P2C, ibc[2][VW], uz, D, nullptr, 1.0, nullptr, 1.0, nullptr, 1.0, 1));
   return "";
+}
+
+// p += phi and Correct_massflux, one lane per velocity component (on g with
+// variable properties, :1609-1613, then q = g / rho, :1915)
+std::string Flow::correct(double sc) {
+  hipLaunchKernelGGL(k_add, grid1(pr.size()), dim3(256), 0, H->stream, pr.p, pcor.p, pr.size(),
+                     mixed ? w32.pr.p : nullptr);
+  Field<double>& ux = thermo ? w64.gx : qx;
+  Field<double>& uy = thermo ? w64.gy : qy;
+  Field<double>& uz = thermo ? w64.gz : qz;
+  const bool st32 = mixed && !thermo;
+  SCHK(fork());
+  SCHK(op<double>(w64, 0, D1_C2P, ibc[0][VP], pcor, ux, nullptr, 1.0, nullptr, 1.0, nullptr, -sc, 1, nullptr, 0.0,
+                  nullptr, 0.0, 0, st32 ? w32.qx.p : nullptr));
+  SCHK(op<double>(w64, 1, D1_C2P, ibc[1][VP], pcor, uy, wall_y ? w64.fby_p : nullptr, 1.0, nullptr, 1.0, nullptr,
+                  -sc, 1, nullptr, 0.0, nullptr, 0.0, 1, st32 ? w32.qy.p : nullptr));
+  SCHK(op<double>(w64, 2, D1_C2P, ibc[2][VP], pcor, uz, nullptr, 1.0, nullptr, 1.0, nullptr, -sc, 1, nullptr, 0.0,
+                  nullptr, 0.0, 2, st32 ? w32.qz.p : nullptr));
+  if (wall_y)
+    hipLaunchKernelGGL(k_enforce_walls, grid1((long)nx * nz), dim3(256), 0, lane_stream(1), uy.p, nx, py, nz,
+                       w64.fby_v, st32 ? w32.qy.p : nullptr);
+  return join();
 }
 
 std::string Flow::substep(int isub) {
@@ -987,25 +1285,11 @@ std::string Flow::substep(int isub) {
   else SCHK(H->poisson->solve(pcor.p, s, coeff));
   // the mixed form's FP32 copies of the new pressure and velocity are
   // stored by the kernels that make them
-  hipLaunchKernelGGL(k_add, grid1(pr.size()), dim3(256), 0, s, pr.p, pcor.p, pr.size(), mixed ? w32.pr.p : nullptr);
-  // Correct_massflux, one lane per velocity component (on g with variable
-  // properties, :1609-1613, then q = g / rho, :1915)
   const double sc = dt * ta[isub] * sigma2p;
-  Field<double>& ux = thermo ? w64.gx : qx;
-  Field<double>& uy = thermo ? w64.gy : qy;
-  Field<double>& uz = thermo ? w64.gz : qz;
-  const bool st32 = mixed && !thermo;
-  SCHK(fork());
-  SCHK(op<double>(w64, 0, D1_C2P, ibc[0][VP], pcor, ux, nullptr, 1.0, nullptr, 1.0, nullptr, -sc, 1, nullptr, 0.0,
-                  nullptr, 0.0, 0, st32 ? w32.qx.p : nullptr));
-  SCHK(op<double>(w64, 1, D1_C2P, ibc[1][VP], pcor, uy, wall_y ? w64.fby_p : nullptr, 1.0, nullptr, 1.0, nullptr,
-                  -sc, 1, nullptr, 0.0, nullptr, 0.0, 1, st32 ? w32.qy.p : nullptr));
-  SCHK(op<double>(w64, 2, D1_C2P, ibc[2][VP], pcor, uz, nullptr, 1.0, nullptr, 1.0, nullptr, -sc, 1, nullptr, 0.0,
-                  nullptr, 0.0, 2, st32 ? w32.qz.p : nullptr));
-  if (wall_y)
-    hipLaunchKernelGGL(k_enforce_walls, grid1((long)nx * nz), dim3(256), 0, lane_stream(1), uy.p, nx, py, nz,
-                       w64.fby_v, st32 ? w32.qy.p : nullptr);
-  SCHK(join());
+  bool fused = false;
+  SCHK(fused_ready(&fused));
+  if (fused) SCHK(correct_fused(sc));
+  else SCHK(correct(sc));
   if (thermo) SCHK(convert_qg(false));
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return std::string("substep: ") + hipGetErrorString(e);

@@ -13,6 +13,7 @@
 #include "../../include/chapsim_hip.h"
 #include "chs_geom.h"
 #include "chs_lineop.h"
+#include "chs_rhs.h"
 
 namespace chs {
 
@@ -39,6 +40,8 @@ struct Handle {
   hipStream_t stream = nullptr;
   std::map<PlanKey, std::unique_ptr<DevPlan<double>>> plans64;
   std::map<PlanKey, std::unique_ptr<DevPlan<float>>> plans32;
+  std::map<PlanKey, std::unique_ptr<DevFusePlan<double>>> fuse64;
+  std::map<PlanKey, std::unique_ptr<DevFusePlan<float>>> fuse32;
   DevBuf io[4];
   std::unique_ptr<Poisson> poisson;
   std::unique_ptr<Flow> flow;
@@ -55,6 +58,10 @@ struct Handle {
   template <typename T>
   std::string plan(int dir, int op, int iacc, const int ibc[2], bool has_fbc, int n_in, int n_out,
                    const DevPlan<T>** out);
+  // the fused form of the same plan (ok false when the line does not have it)
+  template <typename T>
+  std::string fuse_plan(int dir, int op, const int ibc[2], bool has_fbc, int n_in, int n_out, bool short_form,
+                        const DevFusePlan<T>** out);
 };
 
 }  // namespace chs

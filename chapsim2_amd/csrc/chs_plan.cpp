@@ -11,6 +11,7 @@
 // the GPU kernels apply.
 #include "chs_plan.h"
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <mutex>
@@ -530,7 +531,7 @@ void line_rhs_host(const LineGeom& g, Op op, int acc, const int ibc[2], const do
 }
 
 std::string make_line_plan(const LineGeom& g, Op op, int acc, const int ibc0[2], bool has_fbc, int n_in, int n_out,
-                           LinePlan* P, int chunk_rows) {
+                           LinePlan* P, int chunk_rows, int chunks) {
   if (n_out < 8 || n_in < 8) return "line too short (need at least 8 points)";
   if (acc < CD2 || acc > CP6) return "invalid accuracy";
   for (int s = 0; s < 2; ++s)
@@ -629,13 +630,17 @@ std::string make_line_plan(const LineGeom& g, Op op, int acc, const int ibc0[2],
   {
     const int n = n_out;
     p.part_ch = (n <= kChunk * kMaxChunks) ? kChunk : kChunkLong;
-    if (chunk_rows == kChunkLong) p.part_ch = kChunkLong;
+    if (chunks > 0) p.part_ch = chunk_rows;
+    else if (chunk_rows == kChunkLong) p.part_ch = kChunkLong;
     else if (chunk_rows != 0 && chunk_rows != kChunk) return "chunk rows must be kChunk or kChunkLong";
-    int P = (n + p.part_ch - 1) / p.part_ch;
+    if (chunks > 0 && (p.part_ch < 1 || (long)chunks * p.part_ch < n || (long)(chunks - 1) * p.part_ch >= n))
+      return "chunks do not cover the line";
+    int P = chunks > 0 ? chunks : (n + p.part_ch - 1) / p.part_ch;
     if (P < 1) P = 1;
     p.part_P = P;
     p.part_start.resize(P + 1);
-    for (int q = 0; q <= P; ++q) p.part_start[q] = (int)((long)q * n / P);
+    for (int q = 0; q <= P; ++q)
+      p.part_start[q] = chunks > 0 ? std::min(q * p.part_ch, n) : (int)((long)q * n / P);
     for (int q = 0; q < P; ++q)
       if (p.part_start[q + 1] - p.part_start[q] < 2) return "chunk shorter than two rows";
   }
