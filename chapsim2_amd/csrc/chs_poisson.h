@@ -54,9 +54,12 @@ class Poisson {
   double* tw_x64 = nullptr; float* tw_x32 = nullptr;   // twiddles of length nx/2 (cos, sin pairs)
   double* tw_z64 = nullptr; float* tw_z32 = nullptr;   // twiddles of length nz
   double* rot64 = nullptr; float* rot32 = nullptr;     // exp(-2 pi i k / nx), k = 0..nx/2
-  double* ya64 = nullptr; double* yc64 = nullptr;      // y tridiagonal off-diagonals (ny)
-  float* ya32 = nullptr; float* yc32 = nullptr;
-  double* fd64 = nullptr; double* fz64 = nullptr;      // per-mode factors (nxh, nz, ny)
+  int td_chunks = 0;                                   // chunks of the partitioned y solve (0: not used)
+  double* yrow = nullptr;                              // y tridiagonal rows: a, c, b, a + c and its rounding (5 ny)
+  double *xr = nullptr, *zr = nullptr;                 // eigenvalues of kx (nxh) and kz (nz)
+  double* f0 = nullptr;                                // TRID0 factors d, z of the (0, 0) mode (2 ny)
+  double* ya64 = nullptr;                              // longer lines: y lower off-diagonal (ny)
+  double* fd64 = nullptr; double* fz64 = nullptr;      // and per-mode factors (nxh, nz, ny)
   float* fd32 = nullptr; float* fz32 = nullptr;
   void* work = nullptr;                                // complex work (nxh, ny, nz)
   size_t work_bytes = 0;

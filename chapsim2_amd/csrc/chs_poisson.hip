@@ -10,9 +10,9 @@
 //
 // Transforms are LDS-resident Stockham FFTs (radix 4/2/3/5), a workgroup per
 // tile of lines; the x transform packs the real line into nx/2 complex points.
-// The per-mode tridiagonal factors (TRID0's D and pivots, including its
-// singular-pivot rule |Z| <= 1e-10 => last unknown 0) are computed once on the
-// host in TRID0's order and read by the y kernel.
+// The y solves of lines of up to 512 rows are partitioned over the lanes of a
+// workgroup (k_ytdma_part); the mean mode keeps TRID0's order and its
+// singular-pivot rule (|Z| <= 1e-10: last unknown 0) with host-built factors.
 #include "chs_poisson.h"
 
 #include <cmath>
@@ -772,6 +772,202 @@ __global__ void __launch_bounds__(64) k_ytdma(cx<T>* __restrict__ W, int nxh, in
   }
 }
 
+// 1 / d for d finite, normal and non-zero: the hardware reciprocal refined by
+// two Newton steps (within an ulp).
+__device__ __forceinline__ double rcp_nr(double d) {
+  double r = __builtin_amdgcn_rcp(d);
+  r = fma(fma(-d, r, 1.0), r, r);
+  return fma(fma(-d, r, 1.0), r, r);
+}
+
+// The (0, 0) mode with TRID0's factors in TRID0's order and its rule for the
+// last pivot (|Z| <= 1e-10: last unknown 0): which of the two it meets is a
+// matter of rounding, so the host's factors decide.  The line in LDS,
+// one thread's sweeps each for the real and the imaginary part.
+template <typename T>
+__device__ __forceinline__ void ytdma_mean(cx<T>* W, int nxh, int ny, const double* __restrict__ ya,
+                                           const double* __restrict__ f0, double* sa) {
+  // sa: a, d, z, re, im
+  double *sd = sa + ny, *sz = sd + ny, *sr = sz + ny, *si = sr + ny;
+  for (int j = threadIdx.x; j < ny; j += blockDim.x) {
+    sa[j] = ya[j];
+    sd[j] = f0[j];
+    sz[j] = f0[ny + j];
+    const cx<T> v = W[(long)nxh * j];
+    sr[j] = v.re;
+    si[j] = v.im;
+  }
+  __syncthreads();
+  if (threadIdx.x < 2) {  // real and imaginary part
+    double* v = threadIdx.x ? si : sr;
+    double t = v[0] * sz[0];
+    v[0] = t;
+#pragma unroll 8
+    for (int j = 1; j < ny - 1; ++j) {
+      t = (v[j] - t * sa[j]) * sz[j];
+      v[j] = t;
+    }
+    const double zl = sz[ny - 1];
+    t = fabs(zl) > 1.0e-10 ? (v[ny - 1] - t * sa[ny - 1]) / zl : 0.0;
+    v[ny - 1] = t;
+#pragma unroll 8
+    for (int j = ny - 2; j >= 0; --j) {
+      t = v[j] - t * sd[j];
+      v[j] = t;
+    }
+  }
+  __syncthreads();
+  for (int j = threadIdx.x; j < ny; j += blockDim.x) W[(long)nxh * j] = {(T)sr[j], (T)si[j]};
+}
+
+// y tridiagonal of every (kx, kz) mode but (0, 0), partitioned: a workgroup is
+// 32 modes (consecutive kx) x P chunks of at most 16 rows, one lane per mode
+// and chunk, the chunk's rows in registers.  Each lane eliminates its chunk
+// forwards and backwards (which gives the chunk's first and last unknown as
+// functions of its neighbours'), the first 32 lanes solve the modes' reduced
+// systems over the chunks, and each lane finishes its chunk with the
+// neighbours' values.  The spectrum is read and written once and the factors
+// are formed on the way; the one-thread-per-mode sweep below reads and writes
+// the spectrum twice and two factor tables of its size (at 512 x 256 x 512 541
+// us, 5.0 TB/s of 2.7 GB; this one 300 us, 1.08 GB).  All arithmetic is FP64,
+// for FP32 spectra too.
+// The rows are -(a + c + sg) x_j + a x_{j-1} + c x_{j+1} with a, c, sg >= 0, so
+// pivots and couplings are kept as sums of non-negative terms: e is a pivot's
+// part beyond its coupling ahead (c + e is the pivot), g and h what a row's
+// couplings lack of 1.  Nothing cancels, also where sg is small against a and
+// c (the long waves), where pivots formed by differences lose three digits
+// (256 rows, sg = 1/4: against extended precision 4e-16, TRID0's order 5e-13).
+// sg is the row sum of the rounded diagonal TRID0 works on, so both solve the
+// same rows.
+constexpr int kTdRows = 16, kTdModes = 32, kTdChunks = 32;
+template <typename T>
+__global__ void __launch_bounds__(kTdModes * kTdChunks) __attribute__((amdgpu_waves_per_eu(4)))
+    k_ytdma_part(cx<T>* W, int nxh, int ny, long nm, const double* __restrict__ yrow,
+                 const double* __restrict__ xr, const double* __restrict__ zr, const double* __restrict__ f0, int P) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  double* sa = reinterpret_cast<double*>(smem);  // the rows' a, c, b, a + c and its rounding
+  if (blockIdx.x == 0) {
+    ytdma_mean<T>(W, nxh, ny, yrow, f0, sa);
+    return;
+  }
+  double* red = sa + 5 * ny;                     // [10][P][32]
+  const int tid = threadIdx.x, nthr = kTdModes * P;
+  const int lane = tid & (kTdModes - 1), q = tid / kTdModes;
+  const long m0 = (long)(blockIdx.x - 1) * kTdModes + lane;
+  const bool live = m0 < nm && m0 > 0;  // (mode 0 is the first workgroup's)
+  const long m = m0 < nm ? m0 : nm - 1;
+  const long kz = m / nxh, kx = m - kz * nxh;
+  const int s0 = (int)((long)q * ny / P), len = (int)((long)(q + 1) * ny / P) - s0;
+  cx<T>* const Wm = W + kx + (long)nxh * ny * kz + (long)nxh * s0;
+  cx<T> raw[kTdRows];
+#pragma unroll
+  for (int i = 0; i < kTdRows; ++i) raw[i] = Wm[(long)nxh * (i < len ? i : len - 1)];
+  auto rhs = [&](int i) -> cx<double> { return {(double)raw[i].re, (double)raw[i].im}; };
+  const double sx = xr[kx], sz = zr[kz];
+  for (int i = tid; i < 5 * ny; i += nthr) sa[i] = yrow[i];
+  __syncthreads();
+  const double *a = sa + s0, *c = sa + ny + s0, *b = sa + 2 * ny + s0, *sm = sa + 3 * ny + s0, *sl = sa + 4 * ny + s0;
+  // row sum of minus the operator, of its rounded diagonal (exact: a difference
+  // of near values, then the rounding of a + c)
+  auto sg = [&](int i) { return -(((b[i] + sx) + sz) + sm[i]) - sl[i]; };
+  // forwards: last unknown yL + uL L_prev + wL F_next, uL + wL + gL = 1
+  double z[kTdRows];  // 1 / pivot
+  cx<double> t{0.0, 0.0};
+  double u = 0.0, g = 0.0, e = 0.0, zl = 0.0;
+#pragma unroll
+  for (int i = 0; i < kTdRows; ++i) {
+    z[i] = 0.0;
+    if (i < len) {
+      const double si = sg(i);
+      e = i ? si + a[i] * (e * zl) : si + a[0];
+      zl = z[i] = rcp_nr(c[i] + e);
+      t = cscale(csub(cscale(t, i ? a[i] : 0.0), rhs(i)), zl);
+      u = i ? a[i] * u * zl : a[0] * zl;
+      g = (si + (i ? a[i] * g : 0.0)) * zl;
+    }
+  }
+  const int M = P * kTdModes, at = q * kTdModes + lane;
+  red[0 * M + at] = t.re;
+  red[1 * M + at] = t.im;
+  red[2 * M + at] = u;
+  red[3 * M + at] = c[len - 1] * zl;
+  red[4 * M + at] = g;
+  // backwards: first unknown
+  t = {0.0, 0.0};
+  u = g = e = zl = 0.0;
+#pragma unroll
+  for (int i = kTdRows - 1; i >= 0; --i) {
+    if (i < len) {
+      const bool end = i == len - 1;
+      const double si = sg(i);
+      e = end ? si + c[i] : si + c[i] * (e * zl);
+      zl = rcp_nr(a[i] + e);
+      t = cscale(csub(cscale(t, end ? 0.0 : c[i]), rhs(i)), zl);
+      u = end ? c[i] * zl : c[i] * u * zl;
+      g = (si + (end ? 0.0 : c[i] * g)) * zl;
+    }
+  }
+  red[5 * M + at] = t.re;
+  red[6 * M + at] = t.im;
+  red[7 * M + at] = a[0] * zl;
+  red[8 * M + at] = u;
+  red[9 * M + at] = g;
+  __syncthreads();
+  // reduced system per mode: upwards L_{k-1} = al + be F_k (be + h = 1) and
+  // F_k = ga + de F_{k+1}, then back
+  if (q == 0) {
+    cx<double> al{0.0, 0.0};
+    double be = 0.0, h = 1.0;
+    for (int k = 0; k < P; ++k) {
+      const int o = k * kTdModes + lane;
+      const cx<double> yL{red[o], red[M + o]}, yF{red[5 * M + o], red[6 * M + o]};
+      const double uL = red[2 * M + o], wL = red[3 * M + o], gL = red[4 * M + o];
+      const double uF = red[7 * M + o], wF = red[8 * M + o], gF = red[9 * M + o];
+      const double gh = gF + uF * h, id = rcp_nr(wF + gh);
+      const cx<double> ga = cscale(cadd(yF, cscale(al, uF)), id);
+      const double de = wF * id;
+      al = cadd(yL, cscale(cadd(al, cscale(ga, be)), uL));
+      h = gL + uL * (h + be * (gh * id));
+      be = wL + uL * (be * de);
+      red[o] = al.re;
+      red[M + o] = al.im;
+      red[2 * M + o] = be;
+      red[5 * M + o] = ga.re;
+      red[6 * M + o] = ga.im;
+      red[7 * M + o] = de;
+    }
+    cx<double> fn{0.0, 0.0};
+    for (int k = P - 1; k >= 0; --k) {
+      const int o = k * kTdModes + lane;
+      const cx<double> L = cadd({red[o], red[M + o]}, cscale(fn, red[2 * M + o]));
+      fn = cadd({red[5 * M + o], red[6 * M + o]}, cscale(fn, red[7 * M + o]));
+      red[o] = L.re;
+      red[M + o] = L.im;
+      red[5 * M + o] = fn.re;
+      red[6 * M + o] = fn.im;
+    }
+  }
+  __syncthreads();
+  // the chunk with its neighbours' values
+  cx<double> r[kTdRows];
+  cx<double> xl{0.0, 0.0}, xf{0.0, 0.0};
+  if (q > 0) xl = cscale({red[at - kTdModes], red[M + at - kTdModes]}, a[0]);
+  if (q < P - 1) xf = cscale({red[5 * M + at + kTdModes], red[6 * M + at + kTdModes]}, c[len - 1]);
+#pragma unroll
+  for (int i = 0; i < kTdRows; ++i) {
+    cx<double> f = csub(i ? cscale(r[i - 1], a[i]) : xl, rhs(i));
+    if (i == len - 1) f = cadd(f, xf);
+    r[i] = cscale(f, z[i]);
+  }
+#pragma unroll
+  for (int i = kTdRows - 2; i >= 0; --i)
+    if (i < len - 1) r[i] = cadd(r[i], cscale(r[i + 1], c[i] * z[i]));
+  if (!live) return;
+#pragma unroll
+  for (int i = 0; i < kTdRows; ++i)
+    if (i < len) Wm[(long)nxh * i] = {(T)r[i].re, (T)r[i].im};
+}
+
 // Wall-normal mixing of the spectrum by a dense ny x ny matrix:
 //   out(i, g) = s(i, g) * sum_j M(i, j) in(j, g)
 // for every real column g = (kz, c) of the complex spectrum (c = 2 kx + re/im),
@@ -1261,7 +1457,7 @@ __global__ void __launch_bounds__(64 * kMmWaves, 4) k_ymix_mfma(const double* __
 
 Poisson::~Poisson() {
   for (void* p : {(void*)tw_x64, (void*)tw_x32, (void*)tw_z64, (void*)tw_z32, (void*)rot64, (void*)rot32,
-                  (void*)ya64, (void*)yc64, (void*)ya32, (void*)yc32, (void*)fd64, (void*)fz64, (void*)fd32,
+                  (void*)ya64, (void*)yrow, (void*)f0, (void*)xr, (void*)zr, (void*)fd64, (void*)fz64, (void*)fd32,
                   (void*)fz32, work, (void*)V64, (void*)Vi64, (void*)lam64, (void*)lx64, (void*)lz64,
                   (void*)V32, (void*)Vi32, (void*)lam32, (void*)lx32, (void*)lz32, work2, (void*)Ve64,
                   (void*)Vo64, (void*)Vie64, (void*)Vio64, (void*)lame64, (void*)lamo64, (void*)Ve32, (void*)Vo32,
@@ -1351,33 +1547,54 @@ std::string Poisson::create(const Mesh& m, int kind, int iacc, std::unique_ptr<P
   } else {
     return "poisson: periodic y needs the 3-D FFT path";
   }
-  if (!(e = upv(a, &p->ya64)).empty() || !(e = upv(c, &p->yc64)).empty()) return e;
-  // TRID0 factors per mode: fz[j] = 1/(bb_j - a_j d_{j-1}) for j < ny-1 and the
+  // TRID0 factors of one mode: fz[j] = 1/(bb_j - a_j d_{j-1}) for j < ny-1 and the
   // raw last pivot at j = ny-1; fd[j] = c_j * z_j.
-  const long nm = (long)p->nxh * p->nz;
-  std::vector<double> fd((size_t)nm * ny), fz((size_t)nm * ny);
   std::vector<double> bb(ny), d(ny);
-  for (int kz = 0; kz < p->nz; ++kz)
-    for (int kx = 0; kx < p->nxh; ++kx) {
-      const double xr = mode_root(xrt, p->nx, kx), zr = mode_root(zrt, p->nz, kz);
-      for (int j = 0; j < ny; ++j) bb[j] = b[j] + xr / (1.0 * 1.0) + zr;
-      const long mi = kx + (long)p->nxh * kz;
-      double z = 1.0 / bb[0];
-      d[0] = c[0] * z;
-      fz[mi] = z;
-      fd[mi] = d[0];
-      for (int j = 1; j < ny - 1; ++j) {
-        z = 1.0 / (bb[j] - a[j] * d[j - 1]);
-        d[j] = c[j] * z;
-        fz[mi + nm * j] = z;
-        fd[mi + nm * j] = d[j];
-      }
-      z = bb[ny - 1] - a[ny - 1] * d[ny - 2];
-      fz[mi + nm * (ny - 1)] = z;
-      fd[mi + nm * (ny - 1)] = 0.0;
+  auto factors = [&](double xrt_, double zrt_, double* fd, double* fz, long stride) {
+    for (int j = 0; j < ny; ++j) bb[j] = b[j] + xrt_ / (1.0 * 1.0) + zrt_;
+    double z = 1.0 / bb[0];
+    d[0] = c[0] * z;
+    fz[0] = z;
+    fd[0] = d[0];
+    for (int j = 1; j < ny - 1; ++j) {
+      z = 1.0 / (bb[j] - a[j] * d[j - 1]);
+      d[j] = c[j] * z;
+      fz[stride * j] = z;
+      fd[stride * j] = d[j];
     }
-  if (!(e = upv(fd, &p->fd64)).empty() || !(e = upv(fz, &p->fz64)).empty()) return e;
-  if (!(e = upv(fd, &p->fd32)).empty() || !(e = upv(fz, &p->fz32)).empty()) return e;
+    z = bb[ny - 1] - a[ny - 1] * d[ny - 2];
+    fz[stride * (ny - 1)] = z;
+    fd[stride * (ny - 1)] = 0.0;
+  };
+  std::vector<double> mx(p->nxh), mz(p->nz);
+  for (int k = 0; k < p->nxh; ++k) mx[k] = mode_root(xrt, p->nx, k);
+  for (int k = 0; k < p->nz; ++k) mz[k] = mode_root(zrt, p->nz, k);
+  p->td_chunks = (ny + kTdRows - 1) / kTdRows;
+  if (p->td_chunks <= kTdChunks) {
+    std::vector<double> row(a), f0(2 * (size_t)ny), sum(ny), low(ny);
+    for (int j = 0; j < ny; ++j) {  // a + c = sum + low
+      sum[j] = a[j] + c[j];
+      const double t = sum[j] - a[j];
+      low[j] = (a[j] - (sum[j] - t)) + (c[j] - t);
+    }
+    for (const std::vector<double>* v : {&c, &b, &sum, &low}) row.insert(row.end(), v->begin(), v->end());
+    factors(mx[0], mz[0], f0.data(), f0.data() + ny, 1);
+    if (!(e = upv(row, &p->yrow)).empty() || !(e = upv(f0, &p->f0)).empty()) return e;
+    if (!(e = upv(mx, &p->xr)).empty() || !(e = upv(mz, &p->zr)).empty()) return e;
+  } else {
+    // lines beyond the partitioned solve: factor tables of every mode
+    p->td_chunks = 0;
+    if (!(e = upv(a, &p->ya64)).empty()) return e;
+    const long nm = (long)p->nxh * p->nz;
+    std::vector<double> fd((size_t)nm * ny), fz((size_t)nm * ny);
+    for (int kz = 0; kz < p->nz; ++kz)
+      for (int kx = 0; kx < p->nxh; ++kx) {
+        const long mi = kx + (long)p->nxh * kz;
+        factors(mx[kx], mz[kz], &fd[mi], &fz[mi], nm);
+      }
+    if (!(e = upv(fd, &p->fd64)).empty() || !(e = upv(fz, &p->fz64)).empty()) return e;
+    if (!(e = upv(fd, &p->fd32)).empty() || !(e = upv(fz, &p->fz32)).empty()) return e;
+  }
   p->work_bytes = sizeof(double) * 2 * (size_t)p->nxh * ny * p->nz;
   PCHK(hipMalloc(&p->work, p->work_bytes));
   if (!(e = p->tune(false)).empty()) return e;
@@ -1619,7 +1836,14 @@ std::string Poisson::solve_t(T* rhs, hipStream_t s, T in_scale) {
   launch_fft_x<T>(true, rhs, W, nullptr, nx, nlx, rx, twx, rot, in_scale, s);
   launch_fft_s<T>(W, nxh, nz, (long)nxh * ny, ny, (long)nxh, rz, twz, T(-1), s);
   const long nm = (long)nxh * nz;
-  hipLaunchKernelGGL(k_ytdma<T>, dim3((unsigned)((nm + 63) / 64)), dim3(64), 0, s, W, nxh, ny, nz, ya64, fd, fz);
+  if (td_chunks > 0) {
+    // (the first workgroup, the mean mode's, needs 5 ny values: no more)
+    const size_t sh = sizeof(double) * (5 * (size_t)ny + 10 * (size_t)td_chunks * kTdModes);
+    hipLaunchKernelGGL(k_ytdma_part<T>, dim3((unsigned)(1 + (nm + kTdModes - 1) / kTdModes)),
+                       dim3((unsigned)(kTdModes * td_chunks)), sh, s, W, nxh, ny, nm, yrow, xr, zr, f0, td_chunks);
+  } else {
+    hipLaunchKernelGGL(k_ytdma<T>, dim3((unsigned)((nm + 63) / 64)), dim3(64), 0, s, W, nxh, ny, nz, ya64, fd, fz);
+  }
   launch_fft_s<T>(W, nxh, nz, (long)nxh * ny, ny, (long)nxh, rz, twz, T(1), s);
   const T scale = T(1.0 / (double(nx) * double(nz)));
   launch_fft_x<T>(false, nullptr, W, rhs, nx, nlx, rx, twx, rot, scale, s);
