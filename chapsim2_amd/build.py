@@ -27,6 +27,8 @@ SOURCES = [
     "chs_rhs.hip",
     "chs_rhs_x.hip",
     "chs_rhs_yz.hip",
+    "chs_fft64.hip",
+    "chs_fft32.hip",
     "chs_poisson.hip",
     "chs_flow.hip",
     "chs_api.hip",
