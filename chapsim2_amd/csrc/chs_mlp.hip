@@ -10,11 +10,12 @@
 //
 // Kernels: a sampling kernel (uniform h, table interpolation, normalised
 // targets); an inference kernel (one thread per sample, weights staged in LDS
-// as FP32 values of the BF16 copies, read as wave-wide broadcasts); a per-sample
-// backward kernel that recomputes the forward pass and writes the layer
-// deltas transposed ([unit][sample]); deterministic batch reductions for the
-// weight gradients (one thread per gradient entry, fixed summation order);
-// and an Adam update of the FP32 master weights followed by the BF16 rounding.
+// as FP32 values of the BF16 copies, read as wave-wide broadcasts); a training
+// kernel for the forward and backward pass (one lane per unit) that writes the
+// activations and layer deltas transposed ([unit][sample]); and deterministic
+// batch reductions for the weight gradients (tiles of entries, fixed summation
+// order) with the Adam update of the FP32 master weights and the BF16 rounding
+// in their epilogue.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -138,114 +139,255 @@ __global__ void __launch_bounds__(256) k_eval(const uint16_t* __restrict__ p16, 
     if (dst[o]) dst[o][b] = (double)out[o] * nm.sd[o] + nm.mu[o];
 }
 
-// Per-sample backward pass of the mean squared error over B samples x 5
+// Forward and backward pass of the mean squared error over B samples x 5
 // outputs.  Samples are either given (given != 0: sample b of xs / ts) or
-// drawn at random from the training set of N samples.  Writes transposed layer quantities for the
-// batch reductions and one loss partial per block.
-__global__ void __launch_bounds__(128) k_bwd(const uint16_t* __restrict__ p16, const float* __restrict__ xs,
-                                             const float* __restrict__ ts, int N, int B, uint32_t seed,
-                                             int given, float* __restrict__ xb, float* __restrict__ a1T,
-                                             float* __restrict__ a2T, float* __restrict__ dz1T,
-                                             float* __restrict__ dz2T, float* __restrict__ dyT,
-                                             float* __restrict__ lossp) {
-  __shared__ float sp[NP];
-  __shared__ float red[128];
-  stage_params(p16, sp);
-  const int b = blockIdx.x * blockDim.x + threadIdx.x;
+// drawn at random from the training set of N samples.  Writes the layer
+// quantities transposed ([unit][sample], rows of Bp) for k_grad and one loss
+// partial per workgroup.
+//
+// One lane per unit of a layer, kTS samples per wave: lane j keeps row j of W2
+// for the forward pass and column j for the backward pass in registers (128
+// of them, FP32 values of the BF16 copies), and the other layer's values
+// arrive as wave-wide LDS broadcasts of four, each used for one
+// multiply-add.  Every sum runs in one lane over ascending units, as one
+// thread per sample would.  Bound by latency: ~20 k multiply-adds per sample
+// are 4 us of chip time at 65536 samples, but a batch of 4096 is one wave per
+// SIMD.  One thread per sample used 64 waves in all for that batch, each with
+// 16 k multiply-adds and their LDS reads in a row: 81 us, now 12.5.
+constexpr int kTS = 4, kTW = 4, kTSB = kTS * kTW;  // samples per wave, waves, samples per workgroup
+constexpr int kTrainBlocks = 1024;                 // grid limit; workgroups walk over the rest
+static_assert(H1 == 64 && H2 == 64 && kTS * NO <= 64, "one lane per unit");
+
+__device__ __forceinline__ float dot64(const float w[64], const float* __restrict__ v, float z) {
+#pragma unroll
+  for (int i = 0; i < 64; i += 4) {
+    const float4 x = *reinterpret_cast<const float4*>(v + i);
+    z += w[i] * x.x;
+    z += w[i + 1] * x.y;
+    z += w[i + 2] * x.z;
+    z += w[i + 3] * x.w;
+  }
+  return z;
+}
+
+__global__ void __launch_bounds__(64 * kTW) k_bwd(const uint16_t* __restrict__ p16, const float* __restrict__ xs,
+                                                  const float* __restrict__ ts, int N, int B, int Bp, uint32_t seed,
+                                                  int given, float* __restrict__ xb, float* __restrict__ a1T,
+                                                  float* __restrict__ a2T, float* __restrict__ dz1T,
+                                                  float* __restrict__ dz2T, float* __restrict__ dyT,
+                                                  float* __restrict__ lossp) {
+  constexpr int kP = kTSB + 1;
+  __shared__ __align__(16) float ex[kTW][kTS][64];  // a layer's values on their way to the other units
+  __shared__ __align__(16) float w3s[NO][68];
+  __shared__ float dys[kTW][kTS][NO + 1];
+  __shared__ float tr[4][64][kP];
+  __shared__ float red[kTW];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  float wr[64], wc[64], w3[NO];
+#pragma unroll
+  for (int i = 0; i < 64; i += 8) {
+    const uint16_t* q = p16 + OW2 + lane * H1 + i;  // rows of 128 bytes
+    const uint4 v = *reinterpret_cast<const uint4*>(q);
+    const uint32_t u[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      wr[i + 2 * k] = __builtin_bit_cast(float, u[k] << 16);
+      wr[i + 2 * k + 1] = __builtin_bit_cast(float, u[k] & 0xFFFF0000U);
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < 64; ++j) wc[j] = bf2f(p16[OW2 + j * H1 + lane]);
+#pragma unroll
+  for (int o = 0; o < NO; ++o) w3[o] = bf2f(p16[OW3 + o * H2 + lane]);
+  const float w1 = bf2f(p16[OW1 + lane]), c1 = bf2f(p16[OB1 + lane]), c2 = bf2f(p16[OB2 + lane]);
+  const int os = lane / NO, oo = lane % NO;  // sample and output of this lane (lanes below kTS * NO)
+  const bool head = lane < kTS * NO;
+  const float c3 = bf2f(p16[OB3 + oo]);
+  if (w == 0)
+#pragma unroll
+    for (int o = 0; o < NO; ++o) w3s[o][lane] = w3[o];
+  const float sc = 2.0f / (float)(B * NO);
   float lsum = 0.0f;
-  if (b < B) {
-    int s = b;
-    if (!given) s = (int)(mix32(mix32((uint32_t)b * 2246822519U) ^ seed) % (uint32_t)N);
-    const float xv = xs[s];
-    float a1[H1];
+  for (int b0 = blockIdx.x * kTSB; b0 < B; b0 += gridDim.x * kTSB) {
+    const int bw = b0 + w * kTS;  // this wave's first sample
+    auto source = [&](int b) {
+      return given ? b : (int)(mix32(mix32((uint32_t)b * 2246822519U) ^ seed) % (uint32_t)N);
+    };
+    float a1[kTS], a2[kTS], d2[kTS];
 #pragma unroll
-    for (int i = 0; i < H1; ++i) a1[i] = tanhf(sp[OW1 + i] * xv + sp[OB1 + i]);
-    float out[NO];
-#pragma unroll
-    for (int o = 0; o < NO; ++o) out[o] = sp[OB3 + o];
-    for (int j = 0; j < H2; ++j) {
-      float z = sp[OB2 + j];
-#pragma unroll
-      for (int i = 0; i < H1; ++i) z += sp[OW2 + j * H1 + i] * a1[i];
-      const float a2 = tanhf(z);
-      a2T[(long)j * B + b] = a2;
-#pragma unroll
-      for (int o = 0; o < NO; ++o) out[o] += sp[OW3 + o * H2 + j] * a2;
+    for (int k = 0; k < kTS; ++k) {
+      const float xv = bw + k < B ? xs[source(bw + k)] : 0.0f;
+      a1[k] = tanhf(w1 * xv + c1);
+      ex[w][k][lane] = a1[k];
+      if (!given && lane == 0 && bw + k < B) xb[bw + k] = xv;
     }
-    const float sc = 2.0f / (float)(B * NO);
-    float dy[NO];
+    float tv = 0.0f;
+    if (head && bw + os < B) tv = ts[(long)oo * (given ? B : N) + source(bw + os)];
+    __syncthreads();
 #pragma unroll
-    for (int o = 0; o < NO; ++o) {
-      const float e = out[o] - ts[(long)o * (given ? B : N) + s];
+    for (int k = 0; k < kTS; ++k) a2[k] = tanhf(dot64(wr, ex[w][k], c2));
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kTS; ++k) ex[w][k][lane] = a2[k];
+    __syncthreads();
+    if (head) {
+      float out = c3;
+#pragma unroll 4
+      for (int j = 0; j < 64; j += 4) {
+        const float4 x = *reinterpret_cast<const float4*>(&ex[w][os][j]);
+        const float4 y = *reinterpret_cast<const float4*>(&w3s[oo][j]);
+        out += y.x * x.x;
+        out += y.y * x.y;
+        out += y.z * x.z;
+        out += y.w * x.w;
+      }
+      const float e = bw + os < B ? out - tv : 0.0f;
       lsum += e * e;
-      dy[o] = sc * e;
-      dyT[(long)o * B + b] = dy[o];
+      dys[w][os][oo] = sc * e;
     }
-    float da1[H1];
+    __syncthreads();
 #pragma unroll
-    for (int i = 0; i < H1; ++i) da1[i] = 0.0f;
-    for (int j = 0; j < H2; ++j) {
-      const float a2 = a2T[(long)j * B + b];
+    for (int k = 0; k < kTS; ++k) {
       float da2 = 0.0f;
 #pragma unroll
-      for (int o = 0; o < NO; ++o) da2 += sp[OW3 + o * H2 + j] * dy[o];
-      const float dz2 = da2 * (1.0f - a2 * a2);
-      dz2T[(long)j * B + b] = dz2;
-#pragma unroll
-      for (int i = 0; i < H1; ++i) da1[i] += sp[OW2 + j * H1 + i] * dz2;
+      for (int o = 0; o < NO; ++o) da2 += w3[o] * dys[w][k][o];
+      d2[k] = da2 * (1.0f - a2[k] * a2[k]);
+      ex[w][k][lane] = d2[k];
     }
+    __syncthreads();
 #pragma unroll
-    for (int i = 0; i < H1; ++i) {
-      a1T[(long)i * B + b] = a1[i];
-      dz1T[(long)i * B + b] = da1[i] * (1.0f - a1[i] * a1[i]);
+    for (int k = 0; k < kTS; ++k) {
+      const float da1 = dot64(wc, ex[w][k], 0.0f);
+      const int c = w * kTS + k;
+      tr[0][lane][c] = a1[k];
+      tr[1][lane][c] = a2[k];
+      tr[2][lane][c] = da1 * (1.0f - a1[k] * a1[k]);
+      tr[3][lane][c] = d2[k];
     }
-    xb[b] = xv;
-  }
-  red[threadIdx.x] = lsum;
-  __syncthreads();
-  for (int k = blockDim.x / 2; k > 0; k >>= 1) {
-    if ((int)threadIdx.x < k) red[threadIdx.x] += red[threadIdx.x + k];
+    __syncthreads();
+    // (rows of Bp, a multiple of kTSB: whole 64-byte segments)
+    float* const dst[4] = {a1T, a2T, dz1T, dz2T};
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int i = threadIdx.x; i < 64 * kTSB; i += 64 * kTW)
+        dst[q][(long)(i / kTSB) * Bp + b0 + i % kTSB] = tr[q][i / kTSB][i % kTSB];
+    if (threadIdx.x < NO * kTSB) {
+      const int o = threadIdx.x / kTSB, c = threadIdx.x % kTSB;
+      dyT[(long)o * Bp + b0 + c] = dys[c / kTS][c % kTS][o];
+    }
     __syncthreads();
   }
-  if (threadIdx.x == 0) lossp[blockIdx.x] = red[0];
-}
-
-// G[r][c] = sum_b U[r][b] * V[c][b] (V null: V = 1) in a fixed order: one
-// workgroup of 256 threads per gradient entry (r, c) = blockIdx.x; thread t
-// sums b = t, t + 256, ... (coalesced across the workgroup), then a fixed
-// tree in LDS adds the 256 partial sums.
-constexpr int kOuterThreads = 256;
-__global__ void __launch_bounds__(kOuterThreads) k_outer(const float* __restrict__ U, int R, const float* __restrict__ V,
-                                                         int C, int B, float* __restrict__ G) {
-  __shared__ float red[kOuterThreads];
-  const int e = blockIdx.x;
-  const int r = e / C, c = e - r * C;
-  const float* u = U + (long)r * B;
-  const float* v = V ? V + (long)c * B : nullptr;
-  float acc = 0.0f;
-  for (int b = threadIdx.x; b < B; b += kOuterThreads) acc += u[b] * (v ? v[b] : 1.0f);
-  red[threadIdx.x] = acc;
+  for (int k = 32; k > 0; k >>= 1) lsum += __shfl_xor(lsum, k);
+  if (lane == 0) red[w] = lsum;
   __syncthreads();
-  for (int k = kOuterThreads / 2; k > 0; k >>= 1) {
-    if ((int)threadIdx.x < k) red[threadIdx.x] += red[threadIdx.x + k];
-    __syncthreads();
+  if (threadIdx.x == 0) {
+    float t = 0.0f;
+    for (int i = 0; i < kTW; ++i) t += red[i];
+    lossp[blockIdx.x] = t;
   }
-  if (threadIdx.x == 0) G[e] = red[0];
 }
 
-__global__ void k_adam(float* __restrict__ p, const float* __restrict__ g, float* __restrict__ m,
-                       float* __restrict__ v, uint16_t* __restrict__ p16, int n, float lr, float b1, float b2,
-                       float eps, float c1, float c2) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const float gi = g[i];
-  const float mi = b1 * m[i] + (1.0f - b1) * gi;
-  const float vi = b2 * v[i] + (1.0f - b2) * gi * gi;
-  m[i] = mi;
-  v[i] = vi;
-  const float pi = p[i] - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
-  p[i] = pi;
-  p16[i] = f2bf(pi);
+// Adam's update of FP32 master weight i and its BF16 copy
+struct Adam {
+  float *p, *m, *v;
+  uint16_t* p16;
+  float lr, b1, b2, eps, c1, c2;
+};
+
+__device__ __forceinline__ void adam_update(const Adam& a, int i, float gi) {
+  const float mi = a.b1 * a.m[i] + (1.0f - a.b1) * gi;
+  const float vi = a.b2 * a.v[i] + (1.0f - a.b2) * gi * gi;
+  a.m[i] = mi;
+  a.v[i] = vi;
+  const float pi = a.p[i] - a.lr * (mi / a.c1) / (sqrtf(vi / a.c2) + a.eps);
+  a.p[i] = pi;
+  a.p16[i] = f2bf(pi);
+}
+
+// All gradients of a batch, G[r][c] = sum_b U[r][b] * V[c][b], and with
+// STEP the Adam update of their weights.  A workgroup of 256 threads owns a
+// tile of NR x NC entries (and, with ONES, the NR row sums besides): thread t
+// sums b = t, t + 256, ... of every entry of the tile, so a row is read once
+// per tile instead of once per entry, and a fixed tree adds the 256 partial
+// sums of each.  Tiles of 16: 256 of them fill the chip for the 64 x 64
+// layer, and read 8 rows for 16 entries.  With one workgroup per entry and a
+// kernel for each of six arrays and for the update a batch of 4096 took 44 us
+// in seven launches, now 9.2 in one.
+constexpr int kGradThreads = 256;
+
+template <int NR, int NC, bool ONES, bool STEP>
+__device__ __forceinline__ void grad_tile(float* red, float* sum, const float* __restrict__ U,
+                                          const float* __restrict__ V, int B, int Bp, int iw, int ldw, int ib,
+                                          float* __restrict__ G, const Adam& ad) {
+  constexpr int E = NR * NC + (ONES ? NR : 0), ND = NC ? NC : 1;
+  float acc[E];
+#pragma unroll
+  for (int e = 0; e < E; ++e) acc[e] = 0.0f;
+#pragma unroll 4
+  for (int b = threadIdx.x; b < B; b += kGradThreads) {
+    float u[NR], v[ND];
+#pragma unroll
+    for (int r = 0; r < NR; ++r) u[r] = U[(long)r * Bp + b];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) v[c] = V[(long)c * Bp + b];
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+#pragma unroll
+      for (int c = 0; c < NC; ++c) acc[r * NC + c] += u[r] * v[c];
+      if (ONES) acc[NR * NC + r] += u[r];
+    }
+  }
+#pragma unroll
+  for (int e = 0; e < E; ++e) red[e * kGradThreads + threadIdx.x] = acc[e];
+  __syncthreads();
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+#pragma unroll
+  for (int e0 = 0; e0 < E; e0 += 4) {
+    const int e = e0 + w;
+    if (e < E) {
+      const float* q = red + e * kGradThreads + lane;
+      float t = (q[0] + q[128]) + (q[64] + q[192]);
+#pragma unroll
+      for (int k = 32; k > 0; k >>= 1) t += __shfl_down(t, k);
+      if (lane == 0) sum[e] = t;
+    }
+  }
+  __syncthreads();
+  const int e = threadIdx.x;
+  if (e < E) {
+    const int i = e < NR * NC ? iw + (e / ND) * ldw + e % ND : ib + e - NR * NC;
+    if (STEP) adam_update(ad, i, sum[e]);
+    else G[i] = sum[e];
+  }
+}
+
+// blocks: 256 tiles 4 x 4 of W2, 8 of eight rows of W1 with b1, 4 of sixteen
+// entries of b2, 16 of W3 (5 x 4) of which the first has b3
+constexpr int kGradW2 = (H2 / 4) * (H1 / 4), kGradW1 = H1 / 8, kGradB2 = H2 / 16, kGradW3 = H2 / 4;
+constexpr int kGradBlocks = kGradW2 + kGradW1 + kGradB2 + kGradW3;
+
+template <bool STEP>
+__global__ void __launch_bounds__(kGradThreads) k_grad(const float* __restrict__ xb, const float* __restrict__ a1T,
+                                                       const float* __restrict__ a2T, const float* __restrict__ dz1T,
+                                                       const float* __restrict__ dz2T, const float* __restrict__ dyT,
+                                                       int B, int Bp, float* __restrict__ G, Adam ad) {
+  __shared__ float red[25 * kGradThreads];
+  __shared__ float sum[25];
+  int k = blockIdx.x;
+  if (k < kGradW2) {
+    const int r = 4 * (k / (H1 / 4)), c = 4 * (k % (H1 / 4));
+    grad_tile<4, 4, false, STEP>(red, sum, dz2T + (long)r * Bp, a1T + (long)c * Bp, B, Bp, OW2 + r * H1 + c, H1, 0, G,
+                                 ad);
+  } else if ((k -= kGradW2) < kGradW1) {
+    grad_tile<8, 1, true, STEP>(red, sum, dz1T + (long)(8 * k) * Bp, xb, B, Bp, OW1 + 8 * k, 1, OB1 + 8 * k, G, ad);
+  } else if ((k -= kGradW1) < kGradB2) {
+    grad_tile<16, 0, true, STEP>(red, sum, dz2T + (long)(16 * k) * Bp, nullptr, B, Bp, 0, 1, OB2 + 16 * k, G, ad);
+  } else if ((k -= kGradB2) == 0) {
+    grad_tile<NO, 4, true, STEP>(red, sum, dyT, a2T, B, Bp, OW3, H2, OB3, G, ad);
+  } else {
+    grad_tile<NO, 4, false, STEP>(red, sum, dyT, a2T + (long)(4 * k) * Bp, B, Bp, OW3 + 4 * k, H2, 0, G, ad);
+  }
 }
 
 __global__ void k_round(const float* __restrict__ p, uint16_t* __restrict__ q, int n) {
@@ -288,25 +430,28 @@ bool dalloc(chs_mlp* m, T** p, size_t n) {
   return true;
 }
 
-// gradients of the batch (already staged by k_bwd) into m->g32; loss sum
-int reduce_grads(chs_mlp* m, int B, int nblk, float* loss) {
+// forward and backward pass over a batch, then the gradients into m->g32 or,
+// with ad, straight into the weights; loss sum on request
+int batch_pass(chs_mlp* m, const float* xs, const float* ts, int N, int B, uint32_t seed, int given, const Adam* ad,
+               float* loss) {
   hipStream_t s = m->stream;
-  auto outer = [&](const float* U, int R, const float* V, int C, float* G) {
-    hipLaunchKernelGGL(k_outer, dim3(R * C), dim3(kOuterThreads), 0, s, U, R, V, C, B, G);
-  };
-  outer(m->dz1T, H1, m->xb, 1, m->g32 + OW1);
-  outer(m->dz1T, H1, nullptr, 1, m->g32 + OB1);
-  outer(m->dz2T, H2, m->a1T, H1, m->g32 + OW2);
-  outer(m->dz2T, H2, nullptr, 1, m->g32 + OB2);
-  outer(m->dyT, NO, m->a2T, H2, m->g32 + OW3);
-  outer(m->dyT, NO, nullptr, 1, m->g32 + OB3);
+  const int Bp = (B + kTSB - 1) / kTSB * kTSB;
+  const int nblk = Bp / kTSB < kTrainBlocks ? Bp / kTSB : kTrainBlocks;
+  hipLaunchKernelGGL(k_bwd, dim3(nblk), dim3(64 * kTW), 0, s, m->p16, xs, ts, N, B, Bp, seed, given, m->xb, m->a1T,
+                     m->a2T, m->dz1T, m->dz2T, m->dyT, m->lossp);
+  if (ad)
+    hipLaunchKernelGGL(k_grad<true>, dim3(kGradBlocks), dim3(kGradThreads), 0, s, m->xb, m->a1T, m->a2T, m->dz1T,
+                       m->dz2T, m->dyT, B, Bp, m->g32, *ad);
+  else
+    hipLaunchKernelGGL(k_grad<false>, dim3(kGradBlocks), dim3(kGradThreads), 0, s, m->xb, m->a1T, m->a2T, m->dz1T,
+                       m->dz2T, m->dyT, B, Bp, m->g32, Adam{});
   if (loss) {
-    std::vector<float> h(nblk);
-    if (hipMemcpyAsync(h.data(), m->lossp, sizeof(float) * nblk, hipMemcpyDeviceToHost, s) != hipSuccess ||
+    float h[kTrainBlocks];
+    if (hipMemcpyAsync(h, m->lossp, sizeof(float) * nblk, hipMemcpyDeviceToHost, s) != hipSuccess ||
         hipStreamSynchronize(s) != hipSuccess)
       return fail(CHS_EHIP, "loss copy");
     double t = 0.0;
-    for (float v : h) t += v;
+    for (int i = 0; i < nblk; ++i) t += h[i];
     *loss = (float)(t / ((double)B * NO));
   }
   if (hipGetLastError() != hipSuccess) return fail(CHS_EHIP, "gradient kernels");
@@ -565,7 +710,7 @@ int chs_mlp_create(chs_props_t* table, int nsamples, unsigned seed, chs_mlp_t** 
             dalloc(m, &m->xs, nsamples) && dalloc(m, &m->ts, (size_t)NO * nsamples) && dalloc(m, &m->xb, kMaxBatch) &&
             dalloc(m, &m->a1T, (size_t)H1 * kMaxBatch) && dalloc(m, &m->a2T, (size_t)H2 * kMaxBatch) &&
             dalloc(m, &m->dz1T, (size_t)H1 * kMaxBatch) && dalloc(m, &m->dz2T, (size_t)H2 * kMaxBatch) &&
-            dalloc(m, &m->dyT, (size_t)NO * kMaxBatch) && dalloc(m, &m->lossp, kMaxBatch / 128 + 1) &&
+            dalloc(m, &m->dyT, (size_t)NO * kMaxBatch) && dalloc(m, &m->lossp, kTrainBlocks) &&
             dalloc(m, &m->tin, (size_t)NO * kMaxBatch);
   if (!ok) {
     delete m;
@@ -634,10 +779,7 @@ int chs_mlp_grad(chs_mlp_t* m, const float* x, const float* t, int B, float* gra
   if (hipMemcpyAsync(m->tin, tt.data(), sizeof(float) * tt.size(), hipMemcpyHostToDevice, s) != hipSuccess ||
       hipMemcpyAsync(m->xb, x, sizeof(float) * B, hipMemcpyHostToDevice, s) != hipSuccess)
     return fail(CHS_EHIP, "copy in");
-  const int nblk = (B + 127) / 128;
-  hipLaunchKernelGGL(k_bwd, dim3(nblk), dim3(128), 0, s, m->p16, m->xb, m->tin, B, B, 0U, 1, m->xb, m->a1T, m->a2T,
-                     m->dz1T, m->dz2T, m->dyT, m->lossp);
-  int rc = reduce_grads(m, B, nblk, loss);
+  int rc = batch_pass(m, m->xb, m->tin, B, B, 0U, 1, nullptr, loss);
   if (rc != CHS_OK) return rc;
   if (hipMemcpyAsync(grad, m->g32, sizeof(float) * NP, hipMemcpyDeviceToHost, s) != hipSuccess ||
       hipStreamSynchronize(s) != hipSuccess)
@@ -648,18 +790,14 @@ int chs_mlp_grad(chs_mlp_t* m, const float* x, const float* t, int B, float* gra
 int chs_mlp_train(chs_mlp_t* m, int steps, int batch, float lr, float* loss) {
   if (!m || steps < 0 || batch < 1 || batch > kMaxBatch || !(lr > 0.0f)) return fail(CHS_EINVAL, "invalid argument");
   hipStream_t s = m->stream;
-  const int nblk = (batch + 127) / 128;
   const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
   for (int it = 0; it < steps; ++it) {
     ++m->step;
     const uint32_t sd = mix32(m->seed * 747796405U + (uint32_t)m->step);
-    hipLaunchKernelGGL(k_bwd, dim3(nblk), dim3(128), 0, s, m->p16, m->xs, m->ts, m->nsamp, batch, sd, 0, m->xb,
-                       m->a1T, m->a2T, m->dz1T, m->dz2T, m->dyT, m->lossp);
-    int rc = reduce_grads(m, batch, nblk, (loss && it == steps - 1) ? loss : nullptr);
-    if (rc != CHS_OK) return rc;
     const float c1 = 1.0f - std::pow(b1, (float)m->step), c2 = 1.0f - std::pow(b2, (float)m->step);
-    hipLaunchKernelGGL(k_adam, dim3((NP + 255) / 256), dim3(256), 0, s, m->p32, m->g32, m->m32, m->v32, m->p16, NP,
-                       lr, b1, b2, eps, c1, c2);
+    const Adam ad{m->p32, m->m32, m->v32, m->p16, lr, b1, b2, eps, c1, c2};
+    int rc = batch_pass(m, m->xs, m->ts, m->nsamp, batch, sd, 0, &ad, (loss && it == steps - 1) ? loss : nullptr);
+    if (rc != CHS_OK) return rc;
   }
   if (hipGetLastError() != hipSuccess || hipStreamSynchronize(s) != hipSuccess) return fail(CHS_EHIP, "training");
   return CHS_OK;
