@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <cstdint>
 #include <string>
 #include <vector>
 
@@ -19,6 +20,10 @@ struct chs_props {
   double ref[7] = {0, 0, 0, 0, 0, 0, 0};
   std::vector<double> col[8];  // t, d, m, k, b, cp, h, rhoh (non-dimensional)
   double* dev = nullptr;       // 8 columns of n, same order
+  double* rec = nullptr;       // per interval: both ends' k, t, b, cp
+  uint16_t* bins = nullptr;    // bins of the search on rho*h (null: none), nbins + 1 row numbers
+  int nbins = 0, rh_sign = 0;  // their number; 1: the column rises, -1: it falls
+  double bscale = 0;           // bins per unit of rho*h
   int* flag = nullptr;         // out-of-range counter
   void* io = nullptr;          // host-memory staging
   size_t io_bytes = 0;
@@ -29,6 +34,8 @@ struct chs_props {
   bool h_rising = false;         // the h column strictly increases (bisections on h may be skipped)
   ~chs_props() {
     if (dev) (void)hipFree(dev);
+    if (rec) (void)hipFree(rec);
+    if (bins) (void)hipFree(bins);
     if (flag) (void)hipFree(flag);
     if (io) (void)hipFree(io);
     if (stream) (void)hipStreamDestroy(stream);
