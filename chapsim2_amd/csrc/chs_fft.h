@@ -22,6 +22,20 @@ __device__ inline cx<T> cscale(cx<T> a, T s) { return {a.re * s, a.im * s}; }
 template <typename T>
 __device__ inline cx<T> cmuli(cx<T> a, T s) { return {-s * a.im, s * a.re}; }
 
+// a store and a load that do not displace what the L2 holds
+template <typename T>
+__device__ __forceinline__ void st_stream(cx<T>* p, cx<T> v) {
+  typedef T pair __attribute__((ext_vector_type(2)));
+  __builtin_nontemporal_store(pair{v.re, v.im}, reinterpret_cast<pair*>(p));
+}
+
+template <typename T>
+__device__ __forceinline__ cx<T> ld_stream(const cx<T>* p) {
+  typedef T pair __attribute__((ext_vector_type(2)));
+  const pair v = __builtin_nontemporal_load(reinterpret_cast<const pair*>(p));
+  return {v.x, v.y};
+}
+
 constexpr int kTileC = 4096;  // longest line (and complex points per workgroup tile of the general kernels)
 
 struct Radices {

@@ -408,6 +408,23 @@ __global__ void __launch_bounds__(LPW * A) k_fft2_s(cx<T>* __restrict__ W, int n
   }
 }
 
+// Barrier of the threads that share x lines: A threads of one wave where A
+// divides 64, so that waves load, transform and store on their own.  With
+// that, the real lines read and written past the L2's replacement and the
+// spectrum's rows (N + 1 entries, which start anywhere) written in whole cache
+// lines, 131072 x lines of 512 take 294 us forward and 253 inverse (330 and
+// 284); streaming stores of the spectrum itself were slower (326; strided
+// lines 275 against 259).
+template <int A>
+__device__ __forceinline__ void lines_sync() {
+  if constexpr (64 % A == 0) {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  } else {
+    __syncthreads();
+  }
+}
+
 // x forward (real lines of 2N -> spectrum kx = 0..N) in two passes; LPW
 // lines per workgroup, thread = a + A * l (lanes along the line).
 template <typename T, int A, int B, int LPW>
@@ -426,14 +443,14 @@ __global__ void __launch_bounds__(LPW * A) k_fft2_x_fwd(const T* __restrict__ in
 #pragma unroll
   for (int b = 0; b < B; ++b) {
     const int n = a + A * b;
-    v[b] = {src[2 * n] * in_scale, src[2 * n + 1] * in_scale};
+    v[b] = cscale(ld_stream(reinterpret_cast<const cx<T>*>(src) + n), in_scale);
   }
   dft_any<T, B, true>(v);
   twiddle_rows<T, B, true>(v, a, twN);
   cx<T>* lb = buf + l * F::LSL;
 #pragma unroll
   for (int k2 = 0; k2 < B; ++k2) lb[k2 * (A + 1) + a] = v[k2];
-  __syncthreads();
+  lines_sync<A>();
   cx<T> z[F::G * A];  // z[g * A + k1] = Z[(a + A g) + B k1]
 #pragma unroll
   for (int g = 0; g < F::G; ++g) {
@@ -445,16 +462,20 @@ __global__ void __launch_bounds__(LPW * A) k_fft2_x_fwd(const T* __restrict__ in
 #pragma unroll
     for (int k1 = 0; k1 < A; ++k1) z[g * A + k1] = u[k1];
   }
-  __syncthreads();  // pass-2 reads done: the line buffer takes Z in natural order
+  lines_sync<A>();  // pass-2 reads done: the line buffer takes Z in natural order
 #pragma unroll
   for (int g = 0; g < F::G; ++g)
 #pragma unroll
     for (int k1 = 0; k1 < A; ++k1)
       if (a + A * g < B) lb[(a + A * g) + B * k1] = z[g * A + k1];
-  __syncthreads();
+  lines_sync<A>();
   if (!ok) return;
   cx<T>* dst = W + L * nxh;
-  for (int k = a; k < nxh; k += A) {
+  // (stores of whole cache lines; W is 256-byte aligned)
+  const int skew = A % 8 == 0 ? (int)((L * nxh) % A) : 0;
+#pragma unroll 4
+  for (int k = a - skew; k < nxh; k += A) {
+    if (k < 0) continue;
     const cx<T> zk = lb[k % N];
     cx<T> zn = lb[(N - k) % N];
     zn.im = -zn.im;  // conj(Z[N-k])
@@ -490,16 +511,16 @@ __global__ void __launch_bounds__(LPW * A) k_fft2_x_inv(const cx<T>* __restrict_
     const cx<T> od = cmul(csub(xk, xn), r);
     lb[k] = {e.re - od.im, e.im + od.re};  // e + i*o
   }
-  __syncthreads();
+  lines_sync<A>();
   cx<T> v[B];
 #pragma unroll
   for (int b = 0; b < B; ++b) v[b] = lb[a + A * b];
   dft_any<T, B, false>(v);
   twiddle_rows<T, B, false>(v, a, twN);
-  __syncthreads();  // every thread has read its pass-1 input
+  lines_sync<A>();  // every thread has read its pass-1 input
 #pragma unroll
   for (int k2 = 0; k2 < B; ++k2) lb[k2 * (A + 1) + a] = v[k2];
-  __syncthreads();
+  lines_sync<A>();
   T* dst = out + L * (2L * N);
 #pragma unroll
   for (int g = 0; g < F::G; ++g) {
@@ -513,8 +534,7 @@ __global__ void __launch_bounds__(LPW * A) k_fft2_x_inv(const cx<T>* __restrict_
 #pragma unroll
       for (int k1 = 0; k1 < A; ++k1) {
         const int n = k2 + B * k1;
-        dst[2 * n] = u[k1].re * scale;
-        dst[2 * n + 1] = u[k1].im * scale;
+        st_stream(reinterpret_cast<cx<T>*>(dst) + n, cscale(u[k1], scale));
       }
     }
   }
