@@ -98,8 +98,8 @@ std::map<PlanKey, std::unique_ptr<DevFusePlan<float>>>& fuse_map<float>(Handle* 
 
 template <typename T>
 std::string Handle::fuse_plan(int dir, int op, const int ibc[2], bool has_fbc, int n_in, int n_out, bool short_form,
-                              const DevFusePlan<T>** out) {
-  PlanKey key{dir, op, desc.iacc, ibc[0], ibc[1], (has_fbc ? 1 : 0) + (short_form ? 2 : 0), n_in, n_out};
+                              int min_rows, const DevFusePlan<T>** out) {
+  PlanKey key{dir, op, desc.iacc, ibc[0], ibc[1], (has_fbc ? 1 : 0) + (short_form ? 2 : 0) + 4 * min_rows, n_in, n_out};
   auto& mp = fuse_map<T>(this);
   auto it = mp.find(key);
   if (it == mp.end()) {
@@ -109,7 +109,7 @@ std::string Handle::fuse_plan(int dir, int op, const int ibc[2], bool has_fbc, i
       LinePlan lp;
       std::string e = make_line_plan(mesh.line_geom(dir), Op(op), desc.iacc, ibc, has_fbc, n_in, n_out, &lp, ell, P);
       if (!e.empty()) return e;
-      e = upload_fuse_plan<T>(lp, rows, dp.get());
+      e = upload_fuse_plan<T>(lp, rows < min_rows ? min_rows : rows, dp.get());
       if (!e.empty()) return e;
     }
     it = mp.emplace(key, std::move(dp)).first;
@@ -117,8 +117,10 @@ std::string Handle::fuse_plan(int dir, int op, const int ibc[2], bool has_fbc, i
   *out = it->second.get();
   return "";
 }
-template std::string Handle::fuse_plan<double>(int, int, const int[2], bool, int, int, bool, const DevFusePlan<double>**);
-template std::string Handle::fuse_plan<float>(int, int, const int[2], bool, int, int, bool, const DevFusePlan<float>**);
+template std::string Handle::fuse_plan<double>(int, int, const int[2], bool, int, int, bool, int,
+                                                const DevFusePlan<double>**);
+template std::string Handle::fuse_plan<float>(int, int, const int[2], bool, int, int, bool, int,
+                                               const DevFusePlan<float>**);
 template std::string Handle::plan<double>(int, int, int, const int[2], bool, int, int, const DevPlan<double>**);
 template std::string Handle::plan<float>(int, int, int, const int[2], bool, int, int, const DevPlan<float>**);
 

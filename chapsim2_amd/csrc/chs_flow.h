@@ -211,8 +211,9 @@ class Flow {
   // the same on the fused operators (constant properties; chs_rhs.h)
   template <typename T> std::string momentum_fused_t(RhsWork<T>& w, int isub, bool fuse);
   template <typename T> std::string fused_plans(FusedPlans<T>& f, bool* ok);
+  bool grouped() const;  // jobs of one kind share launches (small grids)
   template <typename T>
-  std::string fused_run(int dir, int kind, const DevFusePlan<T>& dp, std::initializer_list<RhsJob<T>> jobs, int lane = 0);
+  std::string fused_run(int kind, std::initializer_list<RhsJob<T>> jobs, int lane = 0);
   std::string fused_ready(bool* ok);  // every operator of the sub-step has its fused plan (decided once)
   std::string divergence_fused(double* d);
   std::string correct(double sc);  // p += phi and the velocity correction

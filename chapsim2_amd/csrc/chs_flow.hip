@@ -932,14 +932,22 @@ std::string Flow::momentum_rhs_t(RhsWork<T>& w, int isub, bool fuse) {
 // ---------------------------------------------------------------------------
 // Grids of up to this many cells take the short chunks.
 constexpr long kShortCells = 1L << 19;
-
+// Grids of up to this many cells put jobs of one kind into one launch.
+constexpr long kGroupCells = 1L << 20;
 template <typename T>
 std::string Flow::fused_plans(FusedPlans<T>& f, bool* ok) {
   const int(*B)[5][2] = ibc;
   bool all = true;
   const bool small = (long)nx * ny * nz <= kShortCells;
+  // y and z lines that share launches share the kernel's chunk length
+  int rows_yz = 0;
+  if ((long)nx * ny * nz <= kGroupCells)
+    for (auto dn : {std::make_pair(1, ny), std::make_pair(1, py), std::make_pair(2, nz), std::make_pair(2, pz)}) {
+      int P, ell, rows;
+      if (fuse_chunks(dn.first, dn.second, small, &P, &ell, &rows)) rows_yz = std::max(rows_yz, rows);
+    }
   auto get = [&](const DevFusePlan<T>** p, int dir, int opk, const int* bc, bool fbc, int n_in, int n_out) {
-    std::string e = H->fuse_plan<T>(dir, opk, bc, fbc, n_in, n_out, small, p);
+    std::string e = H->fuse_plan<T>(dir, opk, bc, fbc, n_in, n_out, small, dir ? rows_yz : 0, p);
     if (e.empty() && !(*p)->ok) all = false;
     return e;
   };
@@ -990,6 +998,8 @@ static RhsJob<T> fused_job(int dir, const Field<T>& A, const Ext3& eo, const Dev
   RhsJob<T> j{};
   const int* a = A.e.n;
   j.A = A.p;
+  j.dir = dir;
+  j.rows = p1.rows;
   j.p1 = p1.k;
   if (p2) j.p2 = p2->k;
   if (dir == 0) {
@@ -1009,17 +1019,17 @@ static RhsJob<T> fused_job(int dir, const Field<T>& A, const Ext3& eo, const Dev
   return j;
 }
 
-// Grids of up to this many cells put jobs of one kind into one launch.
-constexpr long kGroupCells = 1L << 20;
+bool Flow::grouped() const { return (long)nx * ny * nz <= kGroupCells && H->prof_class < 0; }
 
 template <typename T>
-std::string Flow::fused_run(int dir, int kind, const DevFusePlan<T>& dp, std::initializer_list<RhsJob<T>> jobs, int lane) {
+std::string Flow::fused_run(int kind, std::initializer_list<RhsJob<T>> jobs, int lane) {
   const hipStream_t s = lane_stream(lane);
-  const bool group = (long)nx * ny * nz <= kGroupCells && H->prof_class < 0;
+  const bool group = grouped();
   RhsGroup<T> g;
   auto flush = [&]() -> std::string {
     if (!g.n) return "";
     hipEvent_t e0 = nullptr, e1 = nullptr;
+    const int dir = g.job[0].dir, rows = g.job[0].rows;
     const bool timed = (H->prof_class == dir) && H->prof_pair(&e0, &e1);
     if (timed) {
       (void)hipEventRecord(e0, s);
@@ -1034,14 +1044,14 @@ std::string Flow::fused_run(int dir, int kind, const DevFusePlan<T>& dp, std::in
         if (kind == RK_CORRECT) H->prof_bytes += 32.0 * no + (J.out32 ? 4.0 * no : 0.0) + (J.add32 ? 4.0 * no : 0.0);
       }
     }
-    std::string e = dir == 0 ? launch_rhs_x<T>(kind, dp.rows, g, s) : launch_rhs_yz<T>(kind, dp.rows, g, s);
+    std::string e = dir == 0 ? launch_rhs_x<T>(kind, rows, g, s) : launch_rhs_yz<T>(kind, rows, g, s);
     if (timed) (void)hipEventRecord(e1, s);
     g.n = 0;
     return e;
   };
   for (const RhsJob<T>& j : jobs) {
+    if (g.n && (!group || g.n == kGroupJobs || j.rows != g.job[0].rows || !j.dir != !g.job[0].dir)) SCHK(flush());
     g.job[g.n++] = j;
-    if (!group || g.n == kGroupJobs) SCHK(flush());
   }
   return flush();
 }
@@ -1105,22 +1115,24 @@ std::string Flow::momentum_fused_t(RhsWork<T>& w, int isub, bool fuse) {
   auto x_z = single(0, w.qxiz, f.xd_c, Z[0]);
   auto z_y = single(2, w.qyiz, f.zd_c, Y[2]);
   auto y_z = single(1, w.qyiz, f.ys_c, Z[1]);
-  // a small grid runs level by level (few, grouped launches); a large one
-  // follows each flux from its making to its two uses while it is in cache
-  SCHK(fused_run<T>(0, RK_PAIR, *f.xi_c, {xp_v, xp_u, xp_w}));
-  SCHK(fused_run<T>(1, RK_SHEAR, *f.yi_n, {s_xy}));
-  SCHK(fused_run<T>(1, RK_PAIR, *f.yi_n, {yp_w}));
-  SCHK(fused_run<T>(1, RK_PAIR, *f.yi_c, {yp_v}));
-  SCHK(fused_run<T>(2, RK_SHEAR, *f.zi_n, {s_xz, s_yz}));
+  // a small grid runs level by level, in few launches of y and z lines
+  // together: each is a serial chain of some 8 us whatever it holds
+  SCHK(fused_run<T>(RK_PAIR, {xp_v, xp_u, xp_w}));
+  if (grouped()) {
+    SCHK(fused_run<T>(RK_PAIR, {yp_w, yp_v}));
+    SCHK(fused_run<T>(RK_SHEAR, {s_xy, s_xz, s_yz}));
+  } else {
+    SCHK(fused_run<T>(RK_SHEAR, {s_xy}));
+    SCHK(fused_run<T>(RK_PAIR, {yp_w, yp_v}));
+    SCHK(fused_run<T>(RK_SHEAR, {s_xz, s_yz}));
+  }
   if (wall_y) {
     const DevPlan<T>* P = nullptr;
     SCHK(H->plan<T>(1, D1_C2P, H->desc.iacc, ibc[1][VV], true, ny, py, &P));
     SCHK(launch_wall_flux<T>(*P, w.qyiy.e, w.qyiy.p, w.fby_v, r, w.fby_visc, s));
   }
-  SCHK(fused_run<T>(2, RK_DIV, *f.zi_c, {dv}));
-  SCHK(fused_run<T>(0, RK_SINGLE, *f.xd_c, {x_y, x_z}));
-  SCHK(fused_run<T>(1, RK_SINGLE, *f.ys_c, {y_x, y_z}));
-  SCHK(fused_run<T>(2, RK_SINGLE, *f.zd_c, {z_x, z_y}));
+  SCHK(fused_run<T>(RK_DIV, {dv}));
+  SCHK(fused_run<T>(RK_SINGLE, {x_y, x_z, y_x, y_z, z_x, z_y}));
   // each component's own direction, the pressure gradient and the fractional step
   const bool forced = H->desc.idriven == 1;
   const Mesh& m = H->mesh;
@@ -1129,8 +1141,10 @@ std::string Flow::momentum_fused_t(RhsWork<T>& w, int isub, bool fuse) {
   const Field<T>* fl[3] = {&w.qxix, &w.qyiy, &w.qziz};
   const DevFusePlan<T>* pf[3] = {f.xd_n, f.yf_n, f.zd_n};
   const DevFusePlan<T>* pp[3] = {f.xd_n, f.yp_n, f.zd_n};
+  RhsJob<T> fin[3];
   for (int c = 0; c < 3; ++c) {
-    RhsJob<T> j = fused_job<T>(c, *fl[c], w.acc[c][0].e, *pf[c], pp[c]);
+    RhsJob<T>& j = fin[c];
+    j = fused_job<T>(c, *fl[c], w.acc[c][0].e, *pf[c], pp[c]);
     j.A2 = w.pr.p;
     if (c == 1 && wall_y) {
       j.fbc = w.fby_visc;
@@ -1150,10 +1164,9 @@ std::string Flow::momentum_fused_t(RhsWork<T>& w, int isub, bool fuse) {
       j.n2 = ny;
       if (rhs_x_blocks<T>(j) > npartial) return "fused: too many partial sums";
     }
-    SCHK(fused_run<T>(c, RK_FINAL, *pf[c], {j}));
-    if (c == 0 && forced)
-      hipLaunchKernelGGL(k_finish_sum, dim3(1), dim3(1024), 0, s, partial, rhs_x_blocks<T>(j), vol, bulk);
   }
+  SCHK(fused_run<T>(RK_FINAL, {fin[0], fin[1], fin[2]}));
+  if (forced) hipLaunchKernelGGL(k_finish_sum, dim3(1), dim3(1024), 0, s, partial, rhs_x_blocks<T>(fin[0]), vol, bulk);
   bulk_pending = fuse && forced;
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return std::string("momentum_fused: ") + hipGetErrorString(e);
@@ -1167,12 +1180,14 @@ std::string Flow::divergence_fused(double* d) {
                  jz = fused_job<double>(2, qz, D.e, *f64.zd_c);
   jx.out = jy.out = jz.out = d;
   jy.sOut = jz.sOut = 1.0;
-  SCHK(fused_run<double>(0, RK_SINGLE, *f64.xd_c, {jx}));
-  SCHK(fused_run<double>(1, RK_CORRECT, *f64.yd_c, {jy}));
-  return fused_run<double>(2, RK_CORRECT, *f64.zd_c, {jz});
+  SCHK(fused_run<double>(RK_SINGLE, {jx}));
+  SCHK(fused_run<double>(RK_CORRECT, {jy}));
+  return fused_run<double>(RK_CORRECT, {jz});
 }
 
-// Correct_massflux on the fused operators, one lane per component: x also does
+// Correct_massflux on the fused operators.  One stream: side streams overlap
+// nothing on large grids, and their events cost some 40 us per sub-step (ten
+// sub-steps of 64^3 lose 0.5 ms, two steps at 256x128x256 0.1).  x also does
 // p += phi (the increment passes that kernel anyway) and the forcing's bulk
 // correction of qx, y sets the wall values (enforce_velo_from_fbc).
 std::string Flow::correct_fused(double sc) {
@@ -1191,11 +1206,7 @@ std::string Flow::correct_fused(double sc) {
     jy.fbc = w64.fby_p;
     jy.fbw = w64.fby_v;
   }
-  SCHK(fork());
-  SCHK(fused_run<double>(0, RK_CORRECT, *f64.xd_n, {jx}, 0));
-  SCHK(fused_run<double>(1, RK_CORRECT, *f64.yp_n, {jy}, 1));
-  SCHK(fused_run<double>(2, RK_CORRECT, *f64.zd_n, {jz}, 2));
-  return join();
+  return fused_run<double>(RK_CORRECT, {jx, jy, jz});
 }
 
 std::string Flow::refresh_q32() {

@@ -58,10 +58,11 @@ struct Handle {
   template <typename T>
   std::string plan(int dir, int op, int iacc, const int ibc[2], bool has_fbc, int n_in, int n_out,
                    const DevPlan<T>** out);
-  // the fused form of the same plan (ok false when the line does not have it)
+  // the fused form of the same plan (ok false when the line does not have it), its tables laid out for chunks of at
+  // least min_rows
   template <typename T>
   std::string fuse_plan(int dir, int op, const int ibc[2], bool has_fbc, int n_in, int n_out, bool short_form,
-                        const DevFusePlan<T>** out);
+                        int min_rows, const DevFusePlan<T>** out);
 };
 
 }  // namespace chs

@@ -16,11 +16,13 @@
 //  - per momentum component one last operator that solves the normal flux and
 //    the pressure along the component's own direction and finishes the
 //    fractional step (rhs0, the state) in place.
-// Several jobs of one kind can share a launch (RhsGroup), which is what small
-// grids need: their launches are latency.
+// Several jobs of one kind can share a launch (RhsGroup), y and z lines
+// together, which is what small grids need: their launches are latency (ten
+// RK3 steps of 64^3 with y and z apart and the corrections on side streams
+// 7.06 ms, now 4.6).
 // Two RK3 steps at 256x128x256 with the state's copies in and out: FP64 12.86
-// -> 10.01 ms, mixed 9.21 -> 7.44 ms; three of six uneven channels as one graph
-// 15.5 -> 11.0 ms; ten of 64^3 9.7 -> 8.0 ms.  What bounds the large grids is
+// -> 9.95 ms, mixed 9.21 -> 7.35 ms; three of six uneven channels as one graph
+// 15.5 -> 10.4 ms; ten of 64^3 9.7 -> 4.6 ms.  What bounds the large grids is
 // memory: the fields moved per sub-step (about 102 with the projection, 139
 // before) at the rate of a large copy (4.8 TB/s); the small ones are bound by
 // each launch's serial chain (arguments, one round trip to memory, the solve,
@@ -103,6 +105,7 @@ std::string upload_fuse_plan(const LinePlan& p, int rows, DevFusePlan<T>* out);
 //          rows from fbw (each pointer possibly null)
 template <typename T>
 struct RhsJob {
+  int dir, rows;              // direction; the plans' chunk length
   int nlines, e1;             // lines; lines per plane (y: nx; z: nx)
   long is, ips, os, ops;      // element strides along the line and per plane, input and output
   const T *A, *A2, *fbc, *fbc2;
@@ -126,16 +129,17 @@ struct RhsJob {
   int n2;                     // y extent (weight index of a line)
 };
 
-constexpr int kGroupJobs = 3;
+constexpr int kGroupJobs = 4;
 template <typename T>
 struct RhsGroup {
   int n = 0;
+  int P;                      // most chunks of a job (y and z lines)
   int first[kGroupJobs + 1];  // first block of each job
   RhsJob<T> job[kGroupJobs];
 };
 
-// Launch the jobs (all of one kind, along one direction, chunk length `rows`)
-// as one grid.  x lines: periodic, contiguous, n_in = n_out.
+// Launch the jobs (all of one kind, chunk length `rows`) as one grid: x lines
+// (periodic, contiguous, n_in = n_out), or y and z lines in any mixture.
 template <typename T>
 std::string launch_rhs_x(int kind, int rows, RhsGroup<T>& g, hipStream_t s);
 // y and z lines; the jobs' plans have the same number of chunks.

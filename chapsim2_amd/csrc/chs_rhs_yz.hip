@@ -33,16 +33,18 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) 
   const RhsJob<T>& J = G.job[jb];
   const FusePlan<T>& p1 = J.p1;
   const FusePlan<T>& p2 = J.p2;
-  const int Pn = p1.P, nthr = NLW * Pn, tid = threadIdx.x;
+  // (the workgroup has lanes for G.P chunks; those past this job's repeat its last one and store nothing)
+  const int Pn = p1.P, nthr = NLW * G.P, tid = threadIdx.x;
   T* ex1 = reinterpret_cast<T*>(smem_raw);
-  T* ex2 = ex1 + (kTwo ? 2 * NLW * Pn : 0);
-  T* s1 = ex2 + 2 * NLW * Pn;
+  T* ex2 = ex1 + (kTwo ? 2 * NLW * G.P : 0);
+  T* s1 = ex2 + 2 * NLW * G.P;
   T* s2 = s1 + p1.ntab;
   TableLoad<T, 2> t1, t2;
   t1.issue(p1, tid, nthr);
   if constexpr (kTwo) t2.issue(p2, tid, nthr);
   const int lane = tid & (NLW - 1);
-  const int q = NLW == 64 ? __builtin_amdgcn_readfirstlane(tid >> 6) : tid / NLW;
+  const int qw = NLW == 64 ? __builtin_amdgcn_readfirstlane(tid >> 6) : tid / NLW;
+  const int q = qw < Pn ? qw : Pn - 1;
   const int L0 = ((int)blockIdx.x - G.first[jb]) * NLW;
   const int Lr = L0 + lane;
   const bool live = Lr < J.nlines;
@@ -142,6 +144,7 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) 
     }
   }
   if (p1.solve || (kTwo && p2.solve)) __syncthreads();
+  if (!live || qw >= Pn) return;
   if (p1.solve)
     fuse_couple<T, CH>(p1, q, s1 + fuse_cp_at(CH) + q * 2 * fuse_band<T>(CH), s1 + cls,
                        [&](int e) { return ex1[lane + NLW * e]; }, y1);
@@ -150,7 +153,6 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) 
       fuse_couple<T, CH>(p2, q, s2 + fuse_cp_at(CH) + q * 2 * fuse_band<T>(CH), s2 + cls,
                          [&](int e) { return ex2[lane + NLW * e]; }, y2);
   }
-  if (!live) return;
   // metric and Neumann rows
   auto post = [&](const FusePlan<T>& p, const T* sm, const T(&fb)[4], T(&y)[CH]) {
     if (p.met) {
@@ -255,25 +257,25 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) 
 }
 
 template <typename T, int KIND, int CH>
-static void yz_width(bool wide, dim3 g, int P, size_t ex, size_t tab, hipStream_t s, const RhsGroup<T>& G) {
+static void yz_width(int nlw, dim3 g, int P, size_t ex, size_t tab, hipStream_t s, const RhsGroup<T>& G) {
   const size_t shm = sizeof(T) * (ex + tab);
-  if (wide)
+  if (nlw == 64)
     hipLaunchKernelGGL((k_rhs_yz<T, KIND, CH, 64>), g, dim3(64 * P), shm, s, G);
   else
     hipLaunchKernelGGL((k_rhs_yz<T, KIND, CH, 32>), g, dim3(32 * P), shm, s, G);
 }
 
 template <typename T, int CH>
-static void yz_kind(int kind, bool wide, dim3 g, int P, size_t ex, size_t tab, hipStream_t s, const RhsGroup<T>& G) {
+static void yz_kind(int kind, int nlw, dim3 g, int P, size_t ex, size_t tab, hipStream_t s, const RhsGroup<T>& G) {
   switch (kind) {
-    case RK_SINGLE: yz_width<T, RK_SINGLE, CH>(wide, g, P, ex, tab, s, G); break;
-    case RK_PAIR: yz_width<T, RK_PAIR, CH>(wide, g, P, ex, tab, s, G); break;
-    case RK_SHEAR: yz_width<T, RK_SHEAR, CH>(wide, g, P, ex, tab, s, G); break;
+    case RK_SINGLE: yz_width<T, RK_SINGLE, CH>(nlw, g, P, ex, tab, s, G); break;
+    case RK_PAIR: yz_width<T, RK_PAIR, CH>(nlw, g, P, ex, tab, s, G); break;
+    case RK_SHEAR: yz_width<T, RK_SHEAR, CH>(nlw, g, P, ex, tab, s, G); break;
     case RK_CORRECT:
-      if constexpr (sizeof(T) == 8) yz_width<T, RK_CORRECT, CH>(wide, g, P, ex, tab, s, G);
+      if constexpr (sizeof(T) == 8) yz_width<T, RK_CORRECT, CH>(nlw, g, P, ex, tab, s, G);
       break;
-    case RK_DIV: yz_width<T, RK_DIV, CH>(wide, g, P, ex, tab, s, G); break;
-    default: yz_width<T, RK_FINAL, CH>(wide, g, P, ex, tab, s, G); break;
+    case RK_DIV: yz_width<T, RK_DIV, CH>(nlw, g, P, ex, tab, s, G); break;
+    default: yz_width<T, RK_FINAL, CH>(nlw, g, P, ex, tab, s, G); break;
   }
 }
 
@@ -283,15 +285,18 @@ std::string launch_rhs_yz(int kind, int rows, RhsGroup<T>& G, hipStream_t s) {
       (kind == RK_CORRECT && sizeof(T) != 8))
     return "fused yz: bad group";
   const bool two = kind != RK_SINGLE && kind != RK_CORRECT;
-  const int P = G.job[0].p1.P;
+  int P = 0;
+  for (int j = 0; j < G.n; ++j) P = std::max(P, G.job[j].p1.P);
+  if (P < 1 || P > kFuseChunks) return "fused yz: bad chunks";
+  G.P = P;
   const bool wide = rows < 16 ? P <= 16 : P <= 8;
   const int nlw = wide ? 64 : 32;
   size_t tab = 0;
   G.first[0] = 0;
   for (int j = 0; j < G.n; ++j) {
     const RhsJob<T>& J = G.job[j];
-    if (J.p1.P != P || P < 1 || P > kFuseChunks || J.p1.ell > rows) return "fused yz: the group's plans differ in chunks";
-    if (two && (J.p2.P != P || J.p2.ell != J.p1.ell || J.p2.n_in != J.p1.n_in || J.p2.n_out != J.p1.n_out ||
+    if (J.p1.P < 1 || J.rows != rows || J.p1.ell > rows) return "fused yz: the group's plans differ in chunks";
+    if (two && (J.p2.P != J.p1.P || J.p2.ell != J.p1.ell || J.p2.n_in != J.p1.n_in || J.p2.n_out != J.p1.n_out ||
                               J.p2.sh != J.p1.sh || J.p2.wrap != J.p1.wrap))
       return "fused yz: a job's two plans differ in geometry";
     if (J.nlines < 1 || J.e1 < 1) return "fused yz: no lines";
@@ -304,10 +309,10 @@ std::string launch_rhs_yz(int kind, int rows, RhsGroup<T>& G, hipStream_t s) {
   const size_t ex = (size_t)2 * nlw * P * (two ? 2 : 1);
   const dim3 g((unsigned)G.first[G.n]);
   switch (rows) {
-    case 8: yz_kind<T, 8>(kind, wide, g, P, ex, tab, s, G); break;
-    case 9: yz_kind<T, 9>(kind, wide, g, P, ex, tab, s, G); break;
-    case 16: yz_kind<T, 16>(kind, wide, g, P, ex, tab, s, G); break;
-    default: yz_kind<T, 17>(kind, wide, g, P, ex, tab, s, G); break;
+    case 8: yz_kind<T, 8>(kind, nlw, g, P, ex, tab, s, G); break;
+    case 9: yz_kind<T, 9>(kind, nlw, g, P, ex, tab, s, G); break;
+    case 16: yz_kind<T, 16>(kind, nlw, g, P, ex, tab, s, G); break;
+    default: yz_kind<T, 17>(kind, nlw, g, P, ex, tab, s, G); break;
   }
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? "" : std::string("fused yz launch: ") + hipGetErrorString(e);
