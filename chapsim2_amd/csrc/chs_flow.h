@@ -132,8 +132,8 @@ class Flow {
   // (there the energy right-hand side is FP32 like the momentum one)
   EnergyWork<double> e64;
   EnergyWork<float> e32;
-  // mixed form: the FP32 copies of g (w32) were made by the energy sub-step
-  // of this sub-step, so the momentum right-hand side need not remake them
+  // mixed form: the FP32 copies of g (w32) equal the rounded FP64 fields (the
+  // last projection or this sub-step's energy equation stored them)
   bool g32_fresh = false;
   // mixed form: the FP32 copies of h, k, T (e32) and mu (w32) equal the
   // rounded FP64 fields (the last property refresh stored them)
@@ -221,7 +221,7 @@ class Flow {
   FusedPlans<double> f64;
   FusedPlans<float> f32;
   int fused_state = 0;        // 0 not decided, 1 fused, 2 single operators
-  bool bulk_pending = false;  // qx holds q + rhs; the forcing's bulk is subtracted by the x correction
+  bool bulk_pending = false;  // qx (gx) holds q + rhs; the forcing's bulk is subtracted by the x correction
   template <typename T> std::string thermo_first_level(RhsWork<T>& w);
   template <typename T> std::string alloc_thermo_work(RhsWork<T>& w);
   std::string refresh_props();

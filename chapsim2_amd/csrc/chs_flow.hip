@@ -900,15 +900,17 @@ std::string Flow::momentum_rhs_t(RhsWork<T>& w, int isub, bool fuse) {
   const Mesh& m = H->mesh;
   const bool forced = (H->desc.idriven == 1);
   // with fuse, components whose update needs no bulk correction are
-  // updated here (x is, when the flow is forced: the correction needs the
-  // whole volume's sum first)
+  // updated here (x of a forced flow is not: its correction needs the whole
+  // volume's sum first, unless the fused x correction applies it)
+  bool later = false;
+  if (fuse) SCHK(fused_ready(&later));
   Field<T>* rhs0[3] = {&w.mx0, &w.my0, &w.mz0};
   // the updated state: q, or g = rho u with variable properties
   double* qs[3] = {thermo ? w64.gx.p : qx.p, thermo ? w64.gy.p : qy.p, thermo ? w64.gz.p : qz.p};
   for (int c = 0; c < 3; ++c) {
     long n = w.acc[c][0].size();
     double* part = (c == 0 && forced) ? partial : nullptr;
-    double* qf = (fuse && !(c == 0 && forced)) ? qs[c] : nullptr;
+    double* qf = (fuse && (later || !(c == 0 && forced))) ? qs[c] : nullptr;
     const double* fbw = (qf && c == 1 && wall_y) ? w64.fby_v : nullptr;
     hipLaunchKernelGGL(k_combine<T>, grid1(n), dim3(256), 0, lane_stream(c), w.acc[c][0].p, w.acc[c][1].p,
                        w.acc[c][2].p, w.acc[c][3].p, rhs0[c]->p, n, T(tg[isub]), T(tz[isub]), T(ta[isub]), T(dt),
@@ -917,10 +919,11 @@ std::string Flow::momentum_rhs_t(RhsWork<T>& w, int isub, bool fuse) {
   if (forced) {
     int nb = (int)((w.acc[0][0].size() + 255) / 256);
     hipLaunchKernelGGL(k_finish_sum, dim3(1), dim3(1024), 0, lane_stream(0), partial, nb, vol, bulk);
-    if (fuse)
+    if (fuse && !later)
       hipLaunchKernelGGL(k_update<T>, grid1(qx.size()), dim3(256), 0, lane_stream(0), qs[0], w.acc[0][0].p,
                          (const double*)bulk, qx.size(), px, ny, (const double*)nullptr);
   }
+  bulk_pending = forced && later;
   SCHK(join());
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return std::string("momentum_rhs: ") + hipGetErrorString(e);
@@ -987,7 +990,7 @@ std::string Flow::fused_ready(bool* ok) {
     }
     fused_state = same && p64 && p32 ? 1 : 2;
   }
-  *ok = fused_state == 1 && !thermo;
+  *ok = fused_state == 1;
   return "";
 }
 
@@ -1173,11 +1176,15 @@ std::string Flow::momentum_fused_t(RhsWork<T>& w, int isub, bool fuse) {
   return "";
 }
 
-// Divergence of the state on the fused operators.
+// Divergence of q, or of g = rho u with variable properties, on the fused
+// operators.
 std::string Flow::divergence_fused(double* d) {
   Field<double> D{d, Ext3{{nx, ny, nz}}};
-  RhsJob<double> jx = fused_job<double>(0, qx, D.e, *f64.xd_c), jy = fused_job<double>(1, qy, D.e, *f64.yd_c),
-                 jz = fused_job<double>(2, qz, D.e, *f64.zd_c);
+  const Field<double>& ux = thermo ? w64.gx : qx;
+  const Field<double>& uy = thermo ? w64.gy : qy;
+  const Field<double>& uz = thermo ? w64.gz : qz;
+  RhsJob<double> jx = fused_job<double>(0, ux, D.e, *f64.xd_c), jy = fused_job<double>(1, uy, D.e, *f64.yd_c),
+                 jz = fused_job<double>(2, uz, D.e, *f64.zd_c);
   jx.out = jy.out = jz.out = d;
   jy.sOut = jz.sOut = 1.0;
   SCHK(fused_run<double>(RK_SINGLE, {jx}));
@@ -1191,13 +1198,19 @@ std::string Flow::divergence_fused(double* d) {
 // p += phi (the increment passes that kernel anyway) and the forcing's bulk
 // correction of qx, y sets the wall values (enforce_velo_from_fbc).
 std::string Flow::correct_fused(double sc) {
-  RhsJob<double> jx = fused_job<double>(0, pcor, qx.e, *f64.xd_n), jy = fused_job<double>(1, pcor, qy.e, *f64.yp_n),
-                 jz = fused_job<double>(2, pcor, qz.e, *f64.zd_n);
+  Field<double>& ux = thermo ? w64.gx : qx;
+  Field<double>& uy = thermo ? w64.gy : qy;
+  Field<double>& uz = thermo ? w64.gz : qz;
+  RhsJob<double> jx = fused_job<double>(0, pcor, ux.e, *f64.xd_n), jy = fused_job<double>(1, pcor, uy.e, *f64.yp_n),
+                 jz = fused_job<double>(2, pcor, uz.e, *f64.zd_n);
   jx.sOut = jy.sOut = jz.sOut = -sc;
-  jx.out = qx.p; jy.out = qy.p; jz.out = qz.p;
+  jx.out = ux.p; jy.out = uy.p; jz.out = uz.p;
   if (mixed) {
-    jx.out32 = w32.qx.p; jy.out32 = w32.qy.p; jz.out32 = w32.qz.p;
+    jx.out32 = thermo ? w32.gx.p : w32.qx.p;
+    jy.out32 = thermo ? w32.gy.p : w32.qy.p;
+    jz.out32 = thermo ? w32.gz.p : w32.qz.p;
     jx.add32 = w32.pr.p;
+    g32_fresh = thermo;
   }
   jx.bulk = bulk_pending ? bulk : nullptr;
   bulk_pending = false;
@@ -1226,13 +1239,14 @@ std::string Flow::momentum_rhs(int isub, bool fuse) {
   set_lanes();
   bool fused = false;
   SCHK(fused_ready(&fused));
+  fused = fused && !thermo;
   if (!mixed) return fused ? momentum_fused_t<double>(w64, isub, fuse) : momentum_rhs_t<double>(w64, isub, fuse);
   // rounded copies of the state for the FP32 right-hand side, unless the
   // last sub-step left them
   if (!q32_fresh) SCHK(refresh_q32());
   if (thermo) {
     // g and mu change every sub-step (projection, property refresh); the
-    // energy sub-step before this right-hand side has rounded g already
+    // projection or the energy sub-step has mostly rounded g already
     hipStream_t s = H->stream;
     for (auto pr2 : {std::make_pair(&w32.gx, &w64.gx), std::make_pair(&w32.gy, &w64.gy),
                      std::make_pair(&w32.gz, &w64.gz), std::make_pair(&w32.visc, &w64.visc)})
@@ -1659,6 +1673,7 @@ std::string Flow::convert_qg(bool to_g) {
   Field<double>* q[3] = {&qx, &qy, &qz};
   Field<double>* g[3] = {&w64.gx, &w64.gy, &w64.gz};
   Field<float>* q32[3] = {&w32.qx, &w32.qy, &w32.qz};
+  if (to_g) g32_fresh = false;
   for (int c = 0; c < 3; ++c) {
     const long n = q[c]->size();
     if (to_g)
@@ -1694,12 +1709,16 @@ std::string Flow::energy_terms() {
   set_lanes();
   if (!mixed) return energy_terms_t<double>(w64, e64);
   // rounded copies of g (kept for this sub-step's momentum right-hand side)
-  // and, unless the last property refresh stored them, of h, k, T
+  // and of h, k, T, unless the last projection and property refresh stored
+  // them (a captured step rounds g itself: its replays follow any state)
   hipStream_t s = H->stream;
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  FCHK(hipStreamIsCapturing(s, &cs));
+  const bool g32 = g32_fresh && cs == hipStreamCaptureStatusNone;
   for (auto pr2 : {std::make_pair(&w32.gx, &w64.gx), std::make_pair(&w32.gy, &w64.gy),
                    std::make_pair(&w32.gz, &w64.gz), std::make_pair(&e32.hent, &hent),
                    std::make_pair(&e32.kcond, &kcond), std::make_pair(&e32.temp, &temp)})
-    if (!props32_fresh || pr2.first == &w32.gx || pr2.first == &w32.gy || pr2.first == &w32.gz)
+    if (pr2.first == &w32.gx || pr2.first == &w32.gy || pr2.first == &w32.gz ? !g32 : !props32_fresh)
       hipLaunchKernelGGL((k_cvt<float, double>), grid1(pr2.second->size()), dim3(256), 0, s, pr2.first->p,
                          pr2.second->p, pr2.second->size());
   return energy_terms_t<float>(w32, e32);
