@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <initializer_list>
+#include <array>
 #include <string>
 #include <vector>
 
@@ -68,6 +69,7 @@ struct FusedPlans {
   const DevFusePlan<T>*ys_c;         // shear flux to cells
   const DevFusePlan<T>*yf_n;         // normal flux to nodes (wall flux)
   const DevFusePlan<T>*yp_n;         // pressure to nodes
+  const DevFusePlan<T>*yi_m;         // viscosity to nodes (wall values)
 };
 
 // The energy right-hand side's operands in the precision T its operators
@@ -210,6 +212,11 @@ class Flow {
   template <typename T> std::string momentum_rhs_t(RhsWork<T>& w, int isub, bool fuse);
   // the same on the fused operators (constant properties; chs_rhs.h)
   template <typename T> std::string momentum_fused_t(RhsWork<T>& w, int isub, bool fuse);
+  template <typename T> std::string momentum_thermo_t(RhsWork<T>& w, int isub, bool fuse);
+  template <typename T>
+  std::string fluxes_fused_t(RhsWork<T>& w, int isub, bool fuse, std::array<Field<T>*, 3> sh,
+                             std::array<Field<T>*, 3> st);
+  template <typename T> std::string wall_stress(RhsWork<T>& w, const T* conv);
   template <typename T> std::string fused_plans(FusedPlans<T>& f, bool* ok);
   bool grouped() const;  // jobs of one kind share launches (small grids)
   template <typename T>

@@ -235,11 +235,12 @@ __global__ void k_extract_walls(T* __restrict__ pl, const T* __restrict__ a, int
 }
 
 // div and visc wall values (nx,4,nz) from the three wall-plane derivatives
-// (times the wall viscosity mu (nx,4,nz) with variable properties, else 1)
+// (times the wall viscosity mu (nx,4,nz) with variable properties, else 1);
+// with conv, visc becomes the wall rows of the whole flux, conv + r visc
 template <typename T>
 __global__ void k_wall_fbc(T* __restrict__ fdiv, T* __restrict__ fvisc, const T* __restrict__ dxw,
                            const T* __restrict__ dyw, const T* __restrict__ dzw, int n1, int n3,
-                           const T* __restrict__ mu) {
+                           const T* __restrict__ mu, const T* __restrict__ conv, T r) {
   long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= (long)n1 * n3) return;
   long i = t % n1, k = t / n1;
@@ -247,6 +248,7 @@ __global__ void k_wall_fbc(T* __restrict__ fdiv, T* __restrict__ fvisc, const T*
     long p = i + (long)n1 * (s + 2 * k);
     T dv = dxw[p] + dyw[p] + dzw[p];
     T vs = (dyw[p] - T(ONE_THIRD) * dv) * T(2) * (mu ? mu[i + (long)n1 * (s + 4 * k)] : T(1));
+    if (conv) vs = conv[i + (long)n1 * (s + 4 * k)] + r * vs;
     fdiv[i + (long)n1 * (s + 4 * k)] = dv;
     fdiv[i + (long)n1 * (s + 2 + 4 * k)] = dv;
     fvisc[i + (long)n1 * (s + 4 * k)] = vs;
@@ -255,6 +257,99 @@ __global__ void k_wall_fbc(T* __restrict__ fdiv, T* __restrict__ fvisc, const T*
 }
 
 // ---- variable-property kernels ----
+// Momentum fluxes in place of the interpolated velocities they are made of,
+// 16 bytes of each field per thread.  Shear at an edge, for its two uses:
+//   f1 <- -a1 f1 + r mu (d1 + d2), f2 <- -a2 f2 + r mu (d1 + d2),
+// normal at the cell centres: f_i <- -a_i f_i + 2 r mu (d_i - div / 3).
+// Bound by memory: 9 and 13 fields once, where the convective and viscous
+// operators read them again each (as window rows, so with their overlap).
+template <typename T>
+struct ShearFlux {
+  T *f1, *f2;
+  const T *a1, *a2, *d1, *d2, *mu;
+  long n;
+};
+template <typename T>
+struct ShearFluxes {
+  ShearFlux<T> p[3];
+};
+template <typename T>
+struct alignas(16) Vec16 {
+  T v[16 / sizeof(T)];
+};
+template <typename T, typename F>
+__device__ __forceinline__ void each16(long n, F&& f) {
+  constexpr int W = 16 / sizeof(T);
+  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x, nv = n / W;
+  if (t < nv) f(t * W, std::integral_constant<int, W>());
+  else if (t - nv < n - nv * W) f(nv * W + (t - nv), std::integral_constant<int, 1>());
+}
+template <int W, typename T>
+__device__ __forceinline__ void get16(const T* p, T (&v)[W]) {
+  if constexpr (W == 1) v[0] = *p;
+  else {
+    const Vec16<T> x = *reinterpret_cast<const Vec16<T>*>(p);
+#pragma unroll
+    for (int c = 0; c < W; ++c) v[c] = x.v[c];
+  }
+}
+template <int W, typename T>
+__device__ __forceinline__ void put16(T* p, const T (&v)[W]) {
+  if constexpr (W == 1) *p = v[0];
+  else {
+    Vec16<T> x;
+#pragma unroll
+    for (int c = 0; c < W; ++c) x.v[c] = v[c];
+    *reinterpret_cast<Vec16<T>*>(p) = x;
+  }
+}
+
+template <typename T>
+__global__ void __launch_bounds__(256) k_shear_flux(ShearFluxes<T> G, T r) {
+  const ShearFlux<T> S = G.p[blockIdx.y];
+  each16<T>(S.n, [&](long i, auto w) {
+    constexpr int W = decltype(w)::value;
+    T f1[W], f2[W], a1[W], a2[W], d1[W], d2[W], mu[W];
+    get16<W>(S.f1 + i, f1); get16<W>(S.f2 + i, f2); get16<W>(S.a1 + i, a1); get16<W>(S.a2 + i, a2);
+    get16<W>(S.d1 + i, d1); get16<W>(S.d2 + i, d2); get16<W>(S.mu + i, mu);
+#pragma unroll
+    for (int c = 0; c < W; ++c) {
+      const T t = r * (mu[c] * (d1[c] + d2[c]));
+      f1[c] = t - a1[c] * f1[c];
+      f2[c] = t - a2[c] * f2[c];
+    }
+    put16<W>(S.f1 + i, f1);
+    put16<W>(S.f2 + i, f2);
+  });
+}
+
+template <typename T>
+struct NormalFlux {
+  T* f[3];
+  const T *a[3], *d[3], *mu;
+  long n;
+};
+template <typename T>
+__global__ void __launch_bounds__(256) k_normal_flux(NormalFlux<T> S, T r) {
+  each16<T>(S.n, [&](long i, auto w) {
+    constexpr int W = decltype(w)::value;
+    T f[3][W], a[3][W], d[3][W], mu[W];
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      get16<W>(S.f[q] + i, f[q]); get16<W>(S.a[q] + i, a[q]); get16<W>(S.d[q] + i, d[q]);
+    }
+    get16<W>(S.mu + i, mu);
+#pragma unroll
+    for (int c = 0; c < W; ++c) {
+      const T third = ((d[0][c] + d[1][c]) + d[2][c]) * T(1.0 / 3.0);
+#pragma unroll
+      for (int q = 0; q < 3; ++q) f[q][c] = r * (mu[c] * (T(2) * (d[q][c] - third))) - a[q][c] * f[q][c];
+    }
+#pragma unroll
+    for (int q = 0; q < 3; ++q) put16<W>(S.f[q] + i, f[q]);
+  });
+}
+
 template <typename T>
 __global__ void k_fill(T* __restrict__ o, T v, long n) {
   long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -778,6 +873,34 @@ std::string Flow::cov_tau(RhsWork<T>& w, int dir, int opk, const int bc_cov[2], 
   return op<T>(w, dir, opk, bc_tau, ta, out, fbc_tau, ts, tb, tc, nullptr, r, 1, nullptr, T(0), nullptr, T(0), lane);
 }
 
+// y-wall values of the divergence and of the y-normal stress (with conv, the
+// wall rows of its whole flux), from the wall planes of qxiy and qziy and the
+// end rows of qyiy.
+template <typename T>
+std::string Flow::wall_stress(RhsWork<T>& w, const T* conv) {
+  if (!wall_y) return "";
+  const int(*B)[5][2] = ibc;
+  const hipStream_t s = H->stream;
+  const long nf2 = (long)nx * nz;
+  // qxdx at the walls: x-derivative of the wall planes of qxiy
+  hipLaunchKernelGGL(k_extract_walls<T>, grid1((long)px * nz), dim3(256), 0, s, w.plane_a, w.qxiy.p, px, py, nz);
+  Field<T> pa{w.plane_a, Ext3{{px, 2, nz}}}, pb{w.plane_b, Ext3{{nx, 2, nz}}};
+  SCHK(op<T>(w, 0, D1_P2C, B[0][VU], pa, pb, nullptr));
+  // qydy at the walls: y-derivative C2P of qyiy (Dirichlet rows are decoupled)
+  {
+    const DevPlan<T>* P = nullptr;
+    SCHK(H->plan<T>(1, D1_C2P, H->desc.iacc, B[1][VV], true, ny, py, &P));
+    SCHK(launch_wall_rows<T>(*P, w.qyiy.e, w.qyiy.p, w.fby_v, w.plane_c, s));
+  }
+  // qzdz at the walls: z-derivative of the wall planes of qziy
+  hipLaunchKernelGGL(k_extract_walls<T>, grid1((long)nx * pz), dim3(256), 0, s, w.plane_a, w.qziy.p, nx, py, pz);
+  Field<T> pa2{w.plane_a, Ext3{{nx, 2, pz}}}, pd{w.plane_d, Ext3{{nx, 2, nz}}};
+  SCHK(op<T>(w, 2, D1_P2C, B[2][VW], pa2, pd, nullptr));
+  hipLaunchKernelGGL(k_wall_fbc<T>, grid1(nf2), dim3(256), 0, s, w.fby_div, w.fby_visc, w.plane_b, w.plane_c,
+                     w.plane_d, nx, nz, (const T*)(thermo ? w.fby_mu : nullptr), conv, T(rre));
+  return "";
+}
+
 // Compute_momentum_rhs + Calculate_momentum_fractional_step + forcing.
 // Result: dt-scaled rhs in w.acc[c][0]; bulk (if forced) in this->bulk.
 template <typename T>
@@ -811,26 +934,7 @@ std::string Flow::momentum_rhs_t(RhsWork<T>& w, int isub, bool fuse) {
   SCHK(join());
   hipLaunchKernelGGL(k_div3<T>, grid1(w.div.size()), dim3(256), 0, s, w.div.p, w.qxdx.p, w.qydy.p, w.qzdz.p,
                      w.div.size());
-  // ---- y-wall values of the divergence and of the y-normal stress ----
-  if (wall_y) {
-    const long nf2 = (long)nx * nz;
-    // qxdx at the walls: x-derivative of the wall planes of qxiy
-    hipLaunchKernelGGL(k_extract_walls<T>, grid1((long)px * nz), dim3(256), 0, s, w.plane_a, w.qxiy.p, px, py, nz);
-    Field<T> pa{w.plane_a, Ext3{{px, 2, nz}}}, pb{w.plane_b, Ext3{{nx, 2, nz}}};
-    SCHK(op<T>(w, 0, D1_P2C, B[0][VU], pa, pb, nullptr));
-    // qydy at the walls: y-derivative C2P of qyiy (Dirichlet rows are decoupled)
-    {
-      const DevPlan<T>* P = nullptr;
-      SCHK(H->plan<T>(1, D1_C2P, H->desc.iacc, B[1][VV], true, ny, py, &P));
-      SCHK(launch_wall_rows<T>(*P, w.qyiy.e, w.qyiy.p, w.fby_v, w.plane_c, s));
-    }
-    // qzdz at the walls: z-derivative of the wall planes of qziy
-    hipLaunchKernelGGL(k_extract_walls<T>, grid1((long)nx * pz), dim3(256), 0, s, w.plane_a, w.qziy.p, nx, py, pz);
-    Field<T> pa2{w.plane_a, Ext3{{nx, 2, pz}}}, pd{w.plane_d, Ext3{{nx, 2, nz}}};
-    SCHK(op<T>(w, 2, D1_P2C, B[2][VW], pa2, pd, nullptr));
-    hipLaunchKernelGGL(k_wall_fbc<T>, grid1(nf2), dim3(256), 0, s, w.fby_div, w.fby_visc, w.plane_b, w.plane_c,
-                       w.plane_d, nx, nz, (const T*)(thermo ? w.fby_mu : nullptr));
-  }
+  SCHK(wall_stress<T>(w, nullptr));
   const T third = T(-ONE_THIRD), two = T(2);
   const T* fconv = wall_y ? w.fby_conv : nullptr;
   const T* fvisc = wall_y ? w.fby_visc : nullptr;
@@ -900,17 +1004,15 @@ std::string Flow::momentum_rhs_t(RhsWork<T>& w, int isub, bool fuse) {
   const Mesh& m = H->mesh;
   const bool forced = (H->desc.idriven == 1);
   // with fuse, components whose update needs no bulk correction are
-  // updated here (x of a forced flow is not: its correction needs the whole
-  // volume's sum first, unless the fused x correction applies it)
-  bool later = false;
-  if (fuse) SCHK(fused_ready(&later));
+  // updated here (x is, when the flow is forced: the correction needs the
+  // whole volume's sum first)
   Field<T>* rhs0[3] = {&w.mx0, &w.my0, &w.mz0};
   // the updated state: q, or g = rho u with variable properties
   double* qs[3] = {thermo ? w64.gx.p : qx.p, thermo ? w64.gy.p : qy.p, thermo ? w64.gz.p : qz.p};
   for (int c = 0; c < 3; ++c) {
     long n = w.acc[c][0].size();
     double* part = (c == 0 && forced) ? partial : nullptr;
-    double* qf = (fuse && (later || !(c == 0 && forced))) ? qs[c] : nullptr;
+    double* qf = (fuse && !(c == 0 && forced)) ? qs[c] : nullptr;
     const double* fbw = (qf && c == 1 && wall_y) ? w64.fby_v : nullptr;
     hipLaunchKernelGGL(k_combine<T>, grid1(n), dim3(256), 0, lane_stream(c), w.acc[c][0].p, w.acc[c][1].p,
                        w.acc[c][2].p, w.acc[c][3].p, rhs0[c]->p, n, T(tg[isub]), T(tz[isub]), T(ta[isub]), T(dt),
@@ -919,11 +1021,10 @@ std::string Flow::momentum_rhs_t(RhsWork<T>& w, int isub, bool fuse) {
   if (forced) {
     int nb = (int)((w.acc[0][0].size() + 255) / 256);
     hipLaunchKernelGGL(k_finish_sum, dim3(1), dim3(1024), 0, lane_stream(0), partial, nb, vol, bulk);
-    if (fuse && !later)
+    if (fuse)
       hipLaunchKernelGGL(k_update<T>, grid1(qx.size()), dim3(256), 0, lane_stream(0), qs[0], w.acc[0][0].p,
                          (const double*)bulk, qx.size(), px, ny, (const double*)nullptr);
   }
-  bulk_pending = forced && later;
   SCHK(join());
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return std::string("momentum_rhs: ") + hipGetErrorString(e);
@@ -963,6 +1064,9 @@ std::string Flow::fused_plans(FusedPlans<T>& f, bool* ok) {
   SCHK(get(&f.ys_c, 1, D1_P2C, mcov[0][1], false, py, ny));
   SCHK(get(&f.yf_n, 1, D1_C2P, mcov[1][1], wall_y, ny, py));
   SCHK(get(&f.yp_n, 1, D1_C2P, B[1][VP], wall_y, ny, py));
+  int ft[2];
+  for (int q = 0; q < 2; ++q) ft[q] = B[1][VT][q] == BC_NEUMANN ? BC_DIRICHLET : B[1][VT][q];
+  SCHK(get(&f.yi_m, 1, MIDP_C2P, ft, wall_y, ny, py));
   *ok = all;
   return "";
 }
@@ -981,7 +1085,7 @@ std::string Flow::fused_ready(bool* ok) {
     for (int d : {0, 2})
       for (int c = 0; c < 3; ++c) {
         same = same && mcov[c][d][0] == BC_PERIODIC && mcov[c][d][1] == BC_PERIODIC;
-        for (int v : {VU, VV, VW, VP}) same = same && ibc[d][v][0] == BC_PERIODIC && ibc[d][v][1] == BC_PERIODIC;
+        for (int v : {VU, VV, VW, VP, VT}) same = same && ibc[d][v][0] == BC_PERIODIC && ibc[d][v][1] == BC_PERIODIC;
       }
     bool p64 = false, p32 = true;
     if (same) {
@@ -1092,12 +1196,6 @@ std::string Flow::momentum_fused_t(RhsWork<T>& w, int isub, bool fuse) {
     j.r = r;
     return j;
   };
-  auto single = [&](int dir, const Field<T>& A, const DevFusePlan<T>* p, Field<T>& out) {
-    RhsJob<T> j = fused_job<T>(dir, A, out.e, *p);
-    j.out = out.p;
-    return j;
-  };
-  Field<T>*X = w.acc[0], *Y = w.acc[1], *Z = w.acc[2];
   auto xp_u = pair(0, w.qx, f.xi_c, nullptr, f.xd_c, nullptr, w.qxix, w.qxdx);
   auto xp_v = pair(0, w.qy, f.xi_n, nullptr, f.xd_n, nullptr, w.qyix, w.qydx);
   auto xp_w = pair(0, w.qz, f.xi_n, nullptr, f.xd_n, nullptr, w.qzix, w.qzdx);
@@ -1112,12 +1210,6 @@ std::string Flow::momentum_fused_t(RhsWork<T>& w, int isub, bool fuse) {
   dv.o1 = w.qxdx.p; dv.o2 = w.qydy.p; dv.o3 = w.qxix.p; dv.o4 = w.qyiy.p;
   dv.out = w.qziz.p;
   dv.r = r;
-  auto y_x = single(1, w.qxiy, f.ys_c, X[1]);
-  auto x_y = single(0, w.qxiy, f.xd_c, Y[0]);
-  auto z_x = single(2, w.qxiz, f.zd_c, X[2]);
-  auto x_z = single(0, w.qxiz, f.xd_c, Z[0]);
-  auto z_y = single(2, w.qyiz, f.zd_c, Y[2]);
-  auto y_z = single(1, w.qyiz, f.ys_c, Z[1]);
   // a small grid runs level by level, in few launches of y and z lines
   // together: each is a serial chain of some 8 us whatever it holds
   SCHK(fused_run<T>(RK_PAIR, {xp_v, xp_u, xp_w}));
@@ -1135,12 +1227,37 @@ std::string Flow::momentum_fused_t(RhsWork<T>& w, int isub, bool fuse) {
     SCHK(launch_wall_flux<T>(*P, w.qyiy.e, w.qyiy.p, w.fby_v, r, w.fby_visc, s));
   }
   SCHK(fused_run<T>(RK_DIV, {dv}));
-  SCHK(fused_run<T>(RK_SINGLE, {x_y, x_z, y_x, y_z, z_x, z_y}));
+  return fluxes_fused_t<T>(w, isub, fuse, {&w.qxiy, &w.qxiz, &w.qyiz}, {&w.qxiy, &w.qxiz, &w.qyiz});
+}
+
+// The derivatives of the momentum fluxes (shear xy, xz, yz as x, x and y read
+// them in sh, as y, z and z do in st; normal ones in qxix, qyiy, qziz), each
+// component's last one with the pressure gradient and the fractional step.
+template <typename T>
+std::string Flow::fluxes_fused_t(RhsWork<T>& w, int isub, bool fuse, std::array<Field<T>*, 3> sh,
+                                 std::array<Field<T>*, 3> st) {
+  FusedPlans<T>* fp;
+  if constexpr (sizeof(T) == 8) fp = &f64;
+  else fp = &f32;
+  const FusedPlans<T>& f = *fp;
+  const hipStream_t s = H->stream;
+  auto single = [&](int dir, const Field<T>& A, const DevFusePlan<T>* p, Field<T>& out) {
+    RhsJob<T> j = fused_job<T>(dir, A, out.e, *p);
+    j.out = out.p;
+    return j;
+  };
+  Field<T>*X = w.acc[0], *Y = w.acc[1], *Z = w.acc[2];
+  auto y_x = single(1, *sh[0], f.ys_c, X[1]);
+  auto x_y = single(0, *st[0], f.xd_c, Y[0]);
+  auto z_x = single(2, *sh[1], f.zd_c, X[2]);
+  auto x_z = single(0, *st[1], f.xd_c, Z[0]);
+  auto z_y = single(2, *sh[2], f.zd_c, Y[2]);
+  auto y_z = single(1, *st[2], f.ys_c, Z[1]);
   // each component's own direction, the pressure gradient and the fractional step
   const bool forced = H->desc.idriven == 1;
   const Mesh& m = H->mesh;
   Field<T>* r0[3] = {&w.mx0, &w.my0, &w.mz0};
-  const Field<double>* qs[3] = {&qx, &qy, &qz};
+  const Field<double>* qs[3] = {thermo ? &w64.gx : &qx, thermo ? &w64.gy : &qy, thermo ? &w64.gz : &qz};
   const Field<T>* fl[3] = {&w.qxix, &w.qyiy, &w.qziz};
   const DevFusePlan<T>* pf[3] = {f.xd_n, f.yf_n, f.zd_n};
   const DevFusePlan<T>* pp[3] = {f.xd_n, f.yp_n, f.zd_n};
@@ -1168,12 +1285,89 @@ std::string Flow::momentum_fused_t(RhsWork<T>& w, int isub, bool fuse) {
       if (rhs_x_blocks<T>(j) > npartial) return "fused: too many partial sums";
     }
   }
-  SCHK(fused_run<T>(RK_FINAL, {fin[0], fin[1], fin[2]}));
+  if (!thermo) {
+    SCHK(fused_run<T>(RK_SINGLE, {x_y, x_z, y_x, y_z, z_x, z_y}));
+    SCHK(fused_run<T>(RK_FINAL, {fin[0], fin[1], fin[2]}));
+  } else {
+    SCHK(fork());
+    SCHK(fused_run<T>(RK_SINGLE, {y_x, z_x}, 0));
+    SCHK(fused_run<T>(RK_FINAL, {fin[0]}, 0));
+    SCHK(fused_run<T>(RK_SINGLE, {x_y, z_y}, 1));
+    SCHK(fused_run<T>(RK_FINAL, {fin[1]}, 1));
+    SCHK(fused_run<T>(RK_SINGLE, {x_z, y_z}, 2));
+    SCHK(fused_run<T>(RK_FINAL, {fin[2]}, 2));
+    SCHK(join());
+  }
   if (forced) hipLaunchKernelGGL(k_finish_sum, dim3(1), dim3(1024), 0, s, partial, rhs_x_blocks<T>(fin[0]), vol, bulk);
   bulk_pending = fuse && forced;
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return std::string("momentum_fused: ") + hipGetErrorString(e);
   return "";
+}
+
+// The same with variable properties (the is_thermo branches of :347-1480):
+// every first-level operator on its fused plan, the fluxes in one elementwise
+// pass each over the edges and the centres, then as above.
+template <typename T>
+std::string Flow::momentum_thermo_t(RhsWork<T>& w, int isub, bool fuse) {
+  FusedPlans<T>* fp;
+  if constexpr (sizeof(T) == 8) fp = &f64;
+  else fp = &f32;
+  const FusedPlans<T>& f = *fp;
+  const hipStream_t s = H->stream;
+  const T* fu = wall_y ? w.fby_u : nullptr;
+  const T* fv = wall_y ? w.fby_v : nullptr;
+  const T* fw = wall_y ? w.fby_w : nullptr;
+  auto pair = [&](int dir, const Field<T>& A, const DevFusePlan<T>* pi, const T* fi, const DevFusePlan<T>* pd,
+                  const T* fd, Field<T>& oi, Field<T>& od) {
+    RhsJob<T> j = fused_job<T>(dir, A, oi.e, *pi, pd);
+    j.fbc = fi; j.fbc2 = fd;
+    j.out = oi.p; j.out2 = od.p;
+    return j;
+  };
+  auto single = [&](int dir, const Field<T>& A, const DevFusePlan<T>* p, const T* fb, Field<T>& out) {
+    RhsJob<T> j = fused_job<T>(dir, A, out.e, *p);
+    j.fbc = fb;
+    j.out = out.p;
+    return j;
+  };
+  SCHK(fork());
+  SCHK(fused_run<T>(RK_PAIR, {pair(0, w.qx, f.xi_c, nullptr, f.xd_c, nullptr, w.qxix, w.qxdx),
+                              pair(0, w.qy, f.xi_n, nullptr, f.xd_n, nullptr, w.qyix, w.qydx),
+                              pair(0, w.qz, f.xi_n, nullptr, f.xd_n, nullptr, w.qzix, w.qzdx)}, 0));
+  SCHK(fused_run<T>(RK_SINGLE, {single(0, w.gx, f.xi_c, nullptr, w.gxix), single(0, w.gy, f.xi_n, nullptr, w.gyix),
+                                single(0, w.gz, f.xi_n, nullptr, w.gzix), single(0, w.visc, f.xi_n, nullptr, w.mupcc)},
+                    0));
+  SCHK(fused_run<T>(RK_SINGLE, {single(2, w.mupcc, f.zi_n, nullptr, w.muixz)}, 0));
+  SCHK(fused_run<T>(RK_SINGLE, {single(1, w.visc, f.yi_m, wall_y ? w.fby_mwall : nullptr, w.muiy),
+                                single(1, w.gx, f.yi_n, fu, w.gxiy), single(1, w.gy, f.yi_c, fv, w.gyiy),
+                                single(1, w.gz, f.yi_n, fw, w.gziy)}, 1));
+  SCHK(fused_run<T>(RK_SINGLE, {single(0, w.muiy, f.xi_n, nullptr, w.muixy)}, 1));
+  if (wall_y)
+    hipLaunchKernelGGL(k_wall_rows4<T>, grid1((long)nx * nz), dim3(256), 0, lane_stream(1), w.fby_mu, w.muiy.p,
+                       (const T*)nullptr, nx, py, nz);
+  SCHK(fused_run<T>(RK_PAIR, {pair(1, w.qx, f.yi_n, fu, f.yd_n, fu, w.qxiy, w.qxdy),
+                              pair(1, w.qy, f.yi_c, fv, f.yd_c, nullptr, w.qyiy, w.qydy),
+                              pair(1, w.qz, f.yi_n, fw, f.yd_n, fw, w.qziy, w.qzdy)}, 1));
+  SCHK(fused_run<T>(RK_PAIR, {pair(2, w.qx, f.zi_n, nullptr, f.zd_n, nullptr, w.qxiz, w.qxdz),
+                              pair(2, w.qy, f.zi_n, nullptr, f.zd_n, nullptr, w.qyiz, w.qydz),
+                              pair(2, w.qz, f.zi_c, nullptr, f.zd_c, nullptr, w.qziz, w.qzdz)}, 2));
+  SCHK(fused_run<T>(RK_SINGLE, {single(2, w.gx, f.zi_n, nullptr, w.gxiz), single(2, w.gy, f.zi_n, nullptr, w.gyiz),
+                                single(2, w.gz, f.zi_c, nullptr, w.gziz)}, 2));
+  SCHK(join());
+  SCHK(fused_run<T>(RK_SINGLE, {single(2, w.muiy, f.zi_n, nullptr, w.muiyz)}));
+  SCHK(wall_stress<T>(w, w.fby_conv));
+  const ShearFluxes<T> sf{{{w.qxiy.p, w.qyix.p, w.gyix.p, w.gxiy.p, w.qxdy.p, w.qydx.p, w.muixy.p, w.qxiy.size()},
+                           {w.qxiz.p, w.qzix.p, w.gzix.p, w.gxiz.p, w.qxdz.p, w.qzdx.p, w.muixz.p, w.qxiz.size()},
+                           {w.qyiz.p, w.qziy.p, w.gziy.p, w.gyiz.p, w.qzdy.p, w.qydz.p, w.muiyz.p, w.qyiz.size()}}};
+  const NormalFlux<T> nf{{w.qxix.p, w.qyiy.p, w.qziz.p}, {w.gxix.p, w.gyiy.p, w.gziz.p},
+                         {w.qxdx.p, w.qydy.p, w.qzdz.p}, w.visc.p, w.qxix.size()};
+  auto vecs = [](long n) { return n / (16 / (long)sizeof(T)) + 16 / (long)sizeof(T); };
+  const dim3 gs = grid1(vecs(std::max({sf.p[0].n, sf.p[1].n, sf.p[2].n})));
+  hipLaunchKernelGGL(k_shear_flux<T>, dim3(gs.x, 3), dim3(256), 0, s, sf, T(rre));
+  hipLaunchKernelGGL(k_normal_flux<T>, grid1(vecs(nf.n)), dim3(256), 0, s, nf, T(rre));
+  FCHK(hipGetLastError());
+  return fluxes_fused_t<T>(w, isub, fuse, {&w.qxiy, &w.qxiz, &w.qyiz}, {&w.qyix, &w.qzix, &w.qziy});
 }
 
 // Divergence of q, or of g = rho u with variable properties, on the fused
@@ -1239,8 +1433,9 @@ std::string Flow::momentum_rhs(int isub, bool fuse) {
   set_lanes();
   bool fused = false;
   SCHK(fused_ready(&fused));
-  fused = fused && !thermo;
-  if (!mixed) return fused ? momentum_fused_t<double>(w64, isub, fuse) : momentum_rhs_t<double>(w64, isub, fuse);
+  if (!mixed)
+    return !fused ? momentum_rhs_t<double>(w64, isub, fuse)
+                  : thermo ? momentum_thermo_t<double>(w64, isub, fuse) : momentum_fused_t<double>(w64, isub, fuse);
   // rounded copies of the state for the FP32 right-hand side, unless the
   // last sub-step left them
   if (!q32_fresh) SCHK(refresh_q32());
@@ -1255,7 +1450,8 @@ std::string Flow::momentum_rhs(int isub, bool fuse) {
                            pr2.second->p, pr2.second->size());
     g32_fresh = false;
   }
-  const std::string r = fused ? momentum_fused_t<float>(w32, isub, fuse) : momentum_rhs_t<float>(w32, isub, fuse);
+  const std::string r = !fused ? momentum_rhs_t<float>(w32, isub, fuse)
+                               : thermo ? momentum_thermo_t<float>(w32, isub, fuse) : momentum_fused_t<float>(w32, isub, fuse);
   if (fuse) q32_fresh = false;  // the state was updated
   return r;
 }
