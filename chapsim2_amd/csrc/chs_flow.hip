@@ -711,6 +711,11 @@ template <typename T>
 std::string Flow::op(RhsWork<T>& w, int dir, int opk, const int ibc2[2], const Field<T>& A, Field<T>& out,
                      const T* fbc, T sA, const Field<T>* B, T cB, const Field<T>* Cm, T sOut, int accumulate,
                      const Field<T>* D, T cD, const Field<T>* E, T cE, int lane, float* out32) {
+  if (thermo && fused_state == 1 && sA == T(1) && !B && !Cm && !D && sOut == T(1) && !accumulate && !out32) {
+    bool done = false;
+    SCHK(single_fused<T>(dir, opk, ibc2, A, out, fbc, lane, &done));
+    if (done) return "";
+  }
   const DevPlan<T>* P = nullptr;
   SCHK(H->plan<T>(dir, opk, H->desc.iacc, ibc2, fbc != nullptr, A.e.n[dir], out.e.n[dir], &P));
   LineIn<T> in;
@@ -1044,7 +1049,7 @@ std::string Flow::fused_plans(FusedPlans<T>& f, bool* ok) {
   bool all = true;
   const bool small = (long)nx * ny * nz <= kShortCells;
   // y and z lines that share launches share the kernel's chunk length
-  int rows_yz = 0;
+  rows_yz = 0;
   if ((long)nx * ny * nz <= kGroupCells)
     for (auto dn : {std::make_pair(1, ny), std::make_pair(1, py), std::make_pair(2, nz), std::make_pair(2, pz)}) {
       int P, ell, rows;
@@ -1161,6 +1166,23 @@ std::string Flow::fused_run(int kind, std::initializer_list<RhsJob<T>> jobs, int
     g.job[g.n++] = j;
   }
   return flush();
+}
+
+// One plain operator of the heated flow on its fused plan, where it has one
+// (a y or z line of 160 FP32 rows reads and writes at 3 TB/s there, in chunks
+// of 16 rows; at 1.6 in the line kernels' chunks of 32).
+template <typename T>
+std::string Flow::single_fused(int dir, int opk, const int* bc, const Field<T>& A, Field<T>& out, const T* fbc, int lane,
+                               bool* done) {
+  const DevFusePlan<T>* p = nullptr;
+  const bool small = (long)nx * ny * nz <= kShortCells;
+  SCHK(H->fuse_plan<T>(dir, opk, bc, fbc != nullptr, A.e.n[dir], out.e.n[dir], small, dir ? rows_yz : 0, &p));
+  *done = p->ok;
+  if (!p->ok) return "";
+  RhsJob<T> j = fused_job<T>(dir, A, out.e, *p);
+  j.fbc = fbc;
+  j.out = out.p;
+  return fused_run<T>(RK_SINGLE, {j}, lane);
 }
 
 // Compute_momentum_rhs, the fractional step and the forcing on the fused
