@@ -217,11 +217,10 @@ class Flow {
   std::string fluxes_fused_t(RhsWork<T>& w, int isub, bool fuse, std::array<Field<T>*, 3> sh,
                              std::array<Field<T>*, 3> st);
   template <typename T>
-  std::string single_fused(int dir, int opk, const int* bc, const Field<T>& A, Field<T>& out, const T* fbc, int lane,
-                           bool* done);
+  std::string plain_job(int dir, int opk, const int* bc, const Field<T>& A, Field<T>& out, const T* fbc, RhsJob<T>* j,
+                        bool* ok);
   template <typename T> std::string wall_stress(RhsWork<T>& w, const T* conv);
   template <typename T> std::string fused_plans(FusedPlans<T>& f, bool* ok);
-  bool grouped() const;  // jobs of one kind share launches (small grids)
   template <typename T>
   std::string fused_run(int kind, std::initializer_list<RhsJob<T>> jobs, int lane = 0);
   std::string fused_ready(bool* ok);  // every operator of the sub-step has its fused plan (decided once)
@@ -230,7 +229,7 @@ class Flow {
   std::string correct_fused(double sc);
   FusedPlans<double> f64;
   FusedPlans<float> f32;
-  int rows_yz = 0;            // least chunk length of the fused y and z plans (0: each its own)
+  int rows_yz = 0;            // least chunk length of the fused y and z plans
   int fused_state = 0;        // 0 not decided, 1 fused, 2 single operators
   bool bulk_pending = false;  // qx (gx) holds q + rhs; the forcing's bulk is subtracted by the x correction
   template <typename T> std::string thermo_first_level(RhsWork<T>& w);

@@ -712,9 +712,10 @@ std::string Flow::op(RhsWork<T>& w, int dir, int opk, const int ibc2[2], const F
                      const T* fbc, T sA, const Field<T>* B, T cB, const Field<T>* Cm, T sOut, int accumulate,
                      const Field<T>* D, T cD, const Field<T>* E, T cE, int lane, float* out32) {
   if (thermo && fused_state == 1 && sA == T(1) && !B && !Cm && !D && sOut == T(1) && !accumulate && !out32) {
-    bool done = false;
-    SCHK(single_fused<T>(dir, opk, ibc2, A, out, fbc, lane, &done));
-    if (done) return "";
+    RhsJob<T> j{};
+    bool ok = false;
+    SCHK(plain_job<T>(dir, opk, ibc2, A, out, fbc, &j, &ok));
+    if (ok) return fused_run<T>(RK_SINGLE, {j}, lane);
   }
   const DevPlan<T>* P = nullptr;
   SCHK(H->plan<T>(dir, opk, H->desc.iacc, ibc2, fbc != nullptr, A.e.n[dir], out.e.n[dir], &P));
@@ -752,8 +753,10 @@ std::string Flow::op(RhsWork<T>& w, int dir, int opk, const int ibc2[2], const F
 
 void Flow::set_lanes() {
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-  // (launch profiling times each kernel on its own, so it keeps one stream)
-  lanes_on = concurrent && side[0] && H->prof_class < 0 && hipStreamIsCapturing(H->stream, &cs) == hipSuccess &&
+  // (launch profiling times each kernel on its own, so it keeps one stream;
+  // the fused operators fill the chip by themselves and save the lanes' events:
+  // heated step 192x96x160 3.85 ms with them, 3.80 without)
+  lanes_on = concurrent && fused_state != 1 && side[0] && H->prof_class < 0 && hipStreamIsCapturing(H->stream, &cs) == hipSuccess &&
              cs == hipStreamCaptureStatusNone;
 }
 
@@ -1039,10 +1042,9 @@ std::string Flow::momentum_rhs_t(RhsWork<T>& w, int isub, bool fuse) {
 // ---------------------------------------------------------------------------
 // The sub-step on the fused operators (chs_rhs.h)
 // ---------------------------------------------------------------------------
-// Grids of up to this many cells take the short chunks.
+// Grids of up to this many cells take the short chunks (beyond, the long ones
+// are faster: two RK3 steps of 160x96x128 FP64 2.97 ms against 3.29).
 constexpr long kShortCells = 1L << 19;
-// Grids of up to this many cells put jobs of one kind into one launch.
-constexpr long kGroupCells = 1L << 20;
 template <typename T>
 std::string Flow::fused_plans(FusedPlans<T>& f, bool* ok) {
   const int(*B)[5][2] = ibc;
@@ -1050,11 +1052,10 @@ std::string Flow::fused_plans(FusedPlans<T>& f, bool* ok) {
   const bool small = (long)nx * ny * nz <= kShortCells;
   // y and z lines that share launches share the kernel's chunk length
   rows_yz = 0;
-  if ((long)nx * ny * nz <= kGroupCells)
-    for (auto dn : {std::make_pair(1, ny), std::make_pair(1, py), std::make_pair(2, nz), std::make_pair(2, pz)}) {
-      int P, ell, rows;
-      if (fuse_chunks(dn.first, dn.second, small, &P, &ell, &rows)) rows_yz = std::max(rows_yz, rows);
-    }
+  for (auto dn : {std::make_pair(1, ny), std::make_pair(1, py), std::make_pair(2, nz), std::make_pair(2, pz)}) {
+    int P, ell, rows;
+    if (fuse_chunks(dn.first, dn.second, small, &P, &ell, &rows)) rows_yz = std::max(rows_yz, rows);
+  }
   auto get = [&](const DevFusePlan<T>** p, int dir, int opk, const int* bc, bool fbc, int n_in, int n_out) {
     std::string e = H->fuse_plan<T>(dir, opk, bc, fbc, n_in, n_out, small, dir ? rows_yz : 0, p);
     if (e.empty() && !(*p)->ok) all = false;
@@ -1131,12 +1132,13 @@ static RhsJob<T> fused_job(int dir, const Field<T>& A, const Ext3& eo, const Dev
   return j;
 }
 
-bool Flow::grouped() const { return (long)nx * ny * nz <= kGroupCells && H->prof_class < 0; }
-
 template <typename T>
 std::string Flow::fused_run(int kind, std::initializer_list<RhsJob<T>> jobs, int lane) {
   const hipStream_t s = lane_stream(lane);
-  const bool group = grouped();
+  // (launch profiling times each operator; otherwise jobs of one kind share a
+  // launch on any grid: two RK3 steps of 192x96x160 FP64 4.42 -> 4.17 ms, of
+  // 128x96x128 mixed 2.40 -> 2.00, of 256x128x256 9.95 -> 9.79)
+  const bool group = H->prof_class < 0;
   RhsGroup<T> g;
   auto flush = [&]() -> std::string {
     if (!g.n) return "";
@@ -1172,17 +1174,17 @@ std::string Flow::fused_run(int kind, std::initializer_list<RhsJob<T>> jobs, int
 // (a y or z line of 160 FP32 rows reads and writes at 3 TB/s there, in chunks
 // of 16 rows; at 1.6 in the line kernels' chunks of 32).
 template <typename T>
-std::string Flow::single_fused(int dir, int opk, const int* bc, const Field<T>& A, Field<T>& out, const T* fbc, int lane,
-                               bool* done) {
+std::string Flow::plain_job(int dir, int opk, const int* bc, const Field<T>& A, Field<T>& out, const T* fbc, RhsJob<T>* j,
+                            bool* ok) {
   const DevFusePlan<T>* p = nullptr;
   const bool small = (long)nx * ny * nz <= kShortCells;
   SCHK(H->fuse_plan<T>(dir, opk, bc, fbc != nullptr, A.e.n[dir], out.e.n[dir], small, dir ? rows_yz : 0, &p));
-  *done = p->ok;
+  *ok = p->ok;
   if (!p->ok) return "";
-  RhsJob<T> j = fused_job<T>(dir, A, out.e, *p);
-  j.fbc = fbc;
-  j.out = out.p;
-  return fused_run<T>(RK_SINGLE, {j}, lane);
+  *j = fused_job<T>(dir, A, out.e, *p);
+  j->fbc = fbc;
+  j->out = out.p;
+  return "";
 }
 
 // Compute_momentum_rhs, the fractional step and the forcing on the fused
@@ -1232,17 +1234,9 @@ std::string Flow::momentum_fused_t(RhsWork<T>& w, int isub, bool fuse) {
   dv.o1 = w.qxdx.p; dv.o2 = w.qydy.p; dv.o3 = w.qxix.p; dv.o4 = w.qyiy.p;
   dv.out = w.qziz.p;
   dv.r = r;
-  // a small grid runs level by level, in few launches of y and z lines
-  // together: each is a serial chain of some 8 us whatever it holds
-  SCHK(fused_run<T>(RK_PAIR, {xp_v, xp_u, xp_w}));
-  if (grouped()) {
-    SCHK(fused_run<T>(RK_PAIR, {yp_w, yp_v}));
-    SCHK(fused_run<T>(RK_SHEAR, {s_xy, s_xz, s_yz}));
-  } else {
-    SCHK(fused_run<T>(RK_SHEAR, {s_xy}));
-    SCHK(fused_run<T>(RK_PAIR, {yp_w, yp_v}));
-    SCHK(fused_run<T>(RK_SHEAR, {s_xz, s_yz}));
-  }
+  // level by level, in few launches of y and z lines together
+  SCHK(fused_run<T>(RK_PAIR, {xp_v, xp_u, xp_w, yp_w, yp_v}));
+  SCHK(fused_run<T>(RK_SHEAR, {s_xy, s_xz, s_yz}));
   if (wall_y) {
     const DevPlan<T>* P = nullptr;
     SCHK(H->plan<T>(1, D1_C2P, H->desc.iacc, ibc[1][VV], true, ny, py, &P));
@@ -1307,19 +1301,8 @@ std::string Flow::fluxes_fused_t(RhsWork<T>& w, int isub, bool fuse, std::array<
       if (rhs_x_blocks<T>(j) > npartial) return "fused: too many partial sums";
     }
   }
-  if (!thermo) {
-    SCHK(fused_run<T>(RK_SINGLE, {x_y, x_z, y_x, y_z, z_x, z_y}));
-    SCHK(fused_run<T>(RK_FINAL, {fin[0], fin[1], fin[2]}));
-  } else {
-    SCHK(fork());
-    SCHK(fused_run<T>(RK_SINGLE, {y_x, z_x}, 0));
-    SCHK(fused_run<T>(RK_FINAL, {fin[0]}, 0));
-    SCHK(fused_run<T>(RK_SINGLE, {x_y, z_y}, 1));
-    SCHK(fused_run<T>(RK_FINAL, {fin[1]}, 1));
-    SCHK(fused_run<T>(RK_SINGLE, {x_z, y_z}, 2));
-    SCHK(fused_run<T>(RK_FINAL, {fin[2]}, 2));
-    SCHK(join());
-  }
+  SCHK(fused_run<T>(RK_SINGLE, {x_y, x_z, y_x, y_z, z_x, z_y}));
+  SCHK(fused_run<T>(RK_FINAL, {fin[0], fin[1], fin[2]}));
   if (forced) hipLaunchKernelGGL(k_finish_sum, dim3(1), dim3(1024), 0, s, partial, rhs_x_blocks<T>(fin[0]), vol, bulk);
   bulk_pending = fuse && forced;
   hipError_t e = hipGetLastError();
@@ -1353,31 +1336,26 @@ std::string Flow::momentum_thermo_t(RhsWork<T>& w, int isub, bool fuse) {
     j.out = out.p;
     return j;
   };
-  SCHK(fork());
   SCHK(fused_run<T>(RK_PAIR, {pair(0, w.qx, f.xi_c, nullptr, f.xd_c, nullptr, w.qxix, w.qxdx),
                               pair(0, w.qy, f.xi_n, nullptr, f.xd_n, nullptr, w.qyix, w.qydx),
-                              pair(0, w.qz, f.xi_n, nullptr, f.xd_n, nullptr, w.qzix, w.qzdx)}, 0));
-  SCHK(fused_run<T>(RK_SINGLE, {single(0, w.gx, f.xi_c, nullptr, w.gxix), single(0, w.gy, f.xi_n, nullptr, w.gyix),
-                                single(0, w.gz, f.xi_n, nullptr, w.gzix), single(0, w.visc, f.xi_n, nullptr, w.mupcc)},
-                    0));
-  SCHK(fused_run<T>(RK_SINGLE, {single(2, w.mupcc, f.zi_n, nullptr, w.muixz)}, 0));
-  SCHK(fused_run<T>(RK_SINGLE, {single(1, w.visc, f.yi_m, wall_y ? w.fby_mwall : nullptr, w.muiy),
-                                single(1, w.gx, f.yi_n, fu, w.gxiy), single(1, w.gy, f.yi_c, fv, w.gyiy),
-                                single(1, w.gz, f.yi_n, fw, w.gziy)}, 1));
-  SCHK(fused_run<T>(RK_SINGLE, {single(0, w.muiy, f.xi_n, nullptr, w.muixy)}, 1));
-  if (wall_y)
-    hipLaunchKernelGGL(k_wall_rows4<T>, grid1((long)nx * nz), dim3(256), 0, lane_stream(1), w.fby_mu, w.muiy.p,
-                       (const T*)nullptr, nx, py, nz);
-  SCHK(fused_run<T>(RK_PAIR, {pair(1, w.qx, f.yi_n, fu, f.yd_n, fu, w.qxiy, w.qxdy),
+                              pair(0, w.qz, f.xi_n, nullptr, f.xd_n, nullptr, w.qzix, w.qzdx),
+                              pair(1, w.qx, f.yi_n, fu, f.yd_n, fu, w.qxiy, w.qxdy),
+                              pair(2, w.qx, f.zi_n, nullptr, f.zd_n, nullptr, w.qxiz, w.qxdz),
                               pair(1, w.qy, f.yi_c, fv, f.yd_c, nullptr, w.qyiy, w.qydy),
-                              pair(1, w.qz, f.yi_n, fw, f.yd_n, fw, w.qziy, w.qzdy)}, 1));
-  SCHK(fused_run<T>(RK_PAIR, {pair(2, w.qx, f.zi_n, nullptr, f.zd_n, nullptr, w.qxiz, w.qxdz),
                               pair(2, w.qy, f.zi_n, nullptr, f.zd_n, nullptr, w.qyiz, w.qydz),
-                              pair(2, w.qz, f.zi_c, nullptr, f.zd_c, nullptr, w.qziz, w.qzdz)}, 2));
-  SCHK(fused_run<T>(RK_SINGLE, {single(2, w.gx, f.zi_n, nullptr, w.gxiz), single(2, w.gy, f.zi_n, nullptr, w.gyiz),
-                                single(2, w.gz, f.zi_c, nullptr, w.gziz)}, 2));
-  SCHK(join());
-  SCHK(fused_run<T>(RK_SINGLE, {single(2, w.muiy, f.zi_n, nullptr, w.muiyz)}));
+                              pair(1, w.qz, f.yi_n, fw, f.yd_n, fw, w.qziy, w.qzdy),
+                              pair(2, w.qz, f.zi_c, nullptr, f.zd_c, nullptr, w.qziz, w.qzdz)}));
+  SCHK(fused_run<T>(RK_SINGLE, {single(0, w.gx, f.xi_c, nullptr, w.gxix), single(0, w.gy, f.xi_n, nullptr, w.gyix),
+                                single(0, w.gz, f.xi_n, nullptr, w.gzix), single(0, w.visc, f.xi_n, nullptr, w.mupcc),
+                                single(1, w.visc, f.yi_m, wall_y ? w.fby_mwall : nullptr, w.muiy),
+                                single(1, w.gx, f.yi_n, fu, w.gxiy), single(1, w.gy, f.yi_c, fv, w.gyiy),
+                                single(1, w.gz, f.yi_n, fw, w.gziy), single(2, w.gx, f.zi_n, nullptr, w.gxiz),
+                                single(2, w.gy, f.zi_n, nullptr, w.gyiz), single(2, w.gz, f.zi_c, nullptr, w.gziz)}));
+  SCHK(fused_run<T>(RK_SINGLE, {single(0, w.muiy, f.xi_n, nullptr, w.muixy), single(2, w.muiy, f.zi_n, nullptr, w.muiyz),
+                                single(2, w.mupcc, f.zi_n, nullptr, w.muixz)}));
+  if (wall_y)
+    hipLaunchKernelGGL(k_wall_rows4<T>, grid1((long)nx * nz), dim3(256), 0, s, w.fby_mu, w.muiy.p,
+                       (const T*)nullptr, nx, py, nz);
   SCHK(wall_stress<T>(w, w.fby_conv));
   const ShearFluxes<T> sf{{{w.qxiy.p, w.qyix.p, w.gyix.p, w.gxiy.p, w.qxdy.p, w.qydx.p, w.muixy.p, w.qxiy.size()},
                            {w.qxiz.p, w.qzix.p, w.gzix.p, w.gxiz.p, w.qxdz.p, w.qzdx.p, w.muixz.p, w.qxiz.size()},
@@ -1962,26 +1940,54 @@ std::string Flow::energy_terms_t(RhsWork<T>& w, EnergyWork<T>& e) {
                const Field<T>* Cm, T sOut, int acc) {
     return op<T>(w, dir, opk, bc, A, out, fbc, sA, nullptr, one, Cm, sOut, acc, nullptr, T(0), nullptr, T(0), lane);
   };
+  // h, k and dT/dx_i at the faces: on fused plans together, or each in its lane
+  bool faces = fused_state == 1;
+  auto face = [&](int dir, int opk, const int* bc, const Field<T>& A, Field<T>& out, const T* fbc) {
+    RhsJob<T> j{};
+    bool ok = false;
+    const std::string err = plain_job<T>(dir, opk, bc, A, out, fbc, &j, &ok);
+    faces = faces && err.empty() && ok;
+    return j;
+  };
+  if (faces) {
+    const RhsJob<T> jx[3] = {face(0, MIDP_C2P, ftp[0], e.hent, e.hpcc, nullptr),
+                             face(0, MIDP_C2P, ftp[0], e.kcond, e.kpcc, nullptr),
+                             face(0, D1_C2P, ibc[0][VT], e.temp, e.tpcc, nullptr)};
+    const RhsJob<T> jy[3] = {face(1, MIDP_C2P, ftp[1], e.hent, e.hcpc, e.fby_h),
+                             face(1, MIDP_C2P, ftp[1], e.kcond, e.kcpc, e.fby_k),
+                             face(1, D1_C2P, ibc[1][VT], e.temp, e.tcpc, e.fby_t)};
+    const RhsJob<T> jz[3] = {face(2, MIDP_C2P, ftp[2], e.hent, e.hccp, nullptr),
+                             face(2, MIDP_C2P, ftp[2], e.kcond, e.kccp, nullptr),
+                             face(2, D1_C2P, ibc[2][VT], e.temp, e.tccp, nullptr)};
+    if (faces)
+      SCHK(fused_run<T>(RK_SINGLE, {jx[0], jx[1], jx[2], jy[0], jy[1], jz[0], jz[1], jy[2], jz[2]}));
+  }
   SCHK(fork());
   // x
-  SCHK(o(0, 0, MIDP_C2P, ftp[0], e.hent, e.hpcc, nullptr, one, nullptr, one, 0));
-  SCHK(o(0, 0, MIDP_C2P, ftp[0], e.kcond, e.kpcc, nullptr, one, nullptr, one, 0));
+  if (!faces) {
+    SCHK(o(0, 0, MIDP_C2P, ftp[0], e.hent, e.hpcc, nullptr, one, nullptr, one, 0));
+    SCHK(o(0, 0, MIDP_C2P, ftp[0], e.kcond, e.kpcc, nullptr, one, nullptr, one, 0));
+    SCHK(o(0, 0, D1_C2P, ibc[0][VT], e.temp, e.tpcc, nullptr, one, nullptr, one, 0));
+  }
   SCHK(o(0, 0, D1_P2C, econv[0], w.gx, e.ex, nullptr, m1, &e.hpcc, one, 0));
-  SCHK(o(0, 0, D1_C2P, ibc[0][VT], e.temp, e.tpcc, nullptr, one, nullptr, one, 0));
   SCHK(o(0, 0, D1_P2C, edifu[0], e.tpcc, e.ex, nullptr, one, &e.kpcc, r, 1));
   // y
-  SCHK(o(1, 1, MIDP_C2P, ftp[1], e.hent, e.hcpc, e.fby_h, one, nullptr, one, 0));
-  SCHK(o(1, 1, MIDP_C2P, ftp[1], e.kcond, e.kcpc, e.fby_k, one, nullptr, one, 0));
+  if (!faces) {
+    SCHK(o(1, 1, MIDP_C2P, ftp[1], e.hent, e.hcpc, e.fby_h, one, nullptr, one, 0));
+    SCHK(o(1, 1, MIDP_C2P, ftp[1], e.kcond, e.kcpc, e.fby_k, one, nullptr, one, 0));
+    SCHK(o(1, 1, D1_C2P, ibc[1][VT], e.temp, e.tcpc, e.fby_t, one, nullptr, one, 0));
+  }
   SCHK(o(1, 1, D1_P2C, econv[1], w.gy, e.ey, nullptr, m1, &e.hcpc, one, 0));
-  SCHK(o(1, 1, D1_C2P, ibc[1][VT], e.temp, e.tcpc, e.fby_t, one, nullptr, one, 0));
   hipLaunchKernelGGL(k_wall_rows4<T>, grid1((long)nx * nz), dim3(256), 0, lane_stream(1), e.fby_q, e.tcpc.p,
                      (const T*)e.kcpc.p, nx, py, nz);
   SCHK(o(1, 1, D1_P2C, edifu[1], e.tcpc, e.ey, e.fby_q, one, &e.kcpc, r, 1));
   // z
-  SCHK(o(2, 2, MIDP_C2P, ftp[2], e.hent, e.hccp, nullptr, one, nullptr, one, 0));
-  SCHK(o(2, 2, MIDP_C2P, ftp[2], e.kcond, e.kccp, nullptr, one, nullptr, one, 0));
+  if (!faces) {
+    SCHK(o(2, 2, MIDP_C2P, ftp[2], e.hent, e.hccp, nullptr, one, nullptr, one, 0));
+    SCHK(o(2, 2, MIDP_C2P, ftp[2], e.kcond, e.kccp, nullptr, one, nullptr, one, 0));
+    SCHK(o(2, 2, D1_C2P, ibc[2][VT], e.temp, e.tccp, nullptr, one, nullptr, one, 0));
+  }
   SCHK(o(2, 2, D1_P2C, econv[2], w.gz, e.ez, nullptr, m1, &e.hccp, one, 0));
-  SCHK(o(2, 2, D1_C2P, ibc[2][VT], e.temp, e.tccp, nullptr, one, nullptr, one, 0));
   SCHK(o(2, 2, D1_P2C, edifu[2], e.tccp, e.ez, nullptr, one, &e.kccp, r, 1));
   SCHK(join());
   return "";
