@@ -489,6 +489,8 @@ __device__ __forceinline__ short bf16_rne(float x) { return __builtin_bit_cast(s
 // out[0..4] (normalised) of the 16 cells whose normalised inputs the lanes
 // with l%16 = c hold in xv; every lane ends with the outputs of cell l%16.
 // wa: this lane's 16 A operands (W2 blocks), sp: the FP32 parameters in LDS.
+// Outputs O0 to O1 - 1 only.
+template <int O0, int O1>
 __device__ __forceinline__ void mlp16_mfma(const bf16x4 wa[16], const float* __restrict__ sp, float xv, float out[NO]) {
   const int q = (threadIdx.x & 63) >> 4;
   bf16x4 bv[4];
@@ -501,7 +503,7 @@ __device__ __forceinline__ void mlp16_mfma(const bf16x4 wa[16], const float* __r
     }
   }
 #pragma unroll
-  for (int o = 0; o < NO; ++o) out[o] = 0.0f;
+  for (int o = O0; o < O1; ++o) out[o] = 0.0f;
 #pragma unroll
   for (int mt = 0; mt < 4; ++mt) {
     f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -512,11 +514,11 @@ __device__ __forceinline__ void mlp16_mfma(const bf16x4 wa[16], const float* __r
       const int u = 16 * mt + 4 * q + r;
       const float a2 = tanh_fast(acc[r] + sp[OB2 + u]);
 #pragma unroll
-      for (int o = 0; o < NO; ++o) out[o] += sp[OW3 + o * H2 + u] * a2;
+      for (int o = O0; o < O1; ++o) out[o] += sp[OW3 + o * H2 + u] * a2;
     }
   }
 #pragma unroll
-  for (int o = 0; o < NO; ++o) {
+  for (int o = O0; o < O1; ++o) {
     out[o] += __shfl_xor(out[o], 16);
     out[o] += __shfl_xor(out[o], 32);
     out[o] += sp[OB3 + o];
@@ -561,17 +563,23 @@ __global__ void __launch_bounds__(256) k_mlp_from_dh_mfma(const uint16_t* __rest
   const double w1 = (crh[i2] - v) / (crh[i2] - crh[i1]), w2 = 1.0 - w1;
   double h = w1 * ch[i1] + w2 * ch[i2];
   float mine[NO];
-  for (int pass = 0; pass < 2; ++pass) {
-    const float x = (float)((h - nm.xc) / nm.xs);
+  // (the first pass needs the density alone: a fifth of the output layer, 180 -> 174 us for 1.3 M cells)
+  float x = (float)((h - nm.xc) / nm.xs);
 #pragma unroll 1
-    for (int p = 0; p < 4; ++p) {
-      float out[NO];
-      mlp16_mfma(wa, sp, __shfl(x, 16 * p + ci), out);
-      if (q == p)
+  for (int p = 0; p < 4; ++p) {
+    float out[NO];
+    mlp16_mfma<1, 2>(wa, sp, __shfl(x, 16 * p + ci), out);
+    if (q == p) mine[1] = out[1];
+  }
+  h = v / ((double)mine[1] * nm.sd[1] + nm.mu[1]);
+  x = (float)((h - nm.xc) / nm.xs);
+#pragma unroll 1
+  for (int p = 0; p < 4; ++p) {
+    float out[NO];
+    mlp16_mfma<0, NO>(wa, sp, __shfl(x, 16 * p + ci), out);
+    if (q == p)
 #pragma unroll
-        for (int o = 0; o < NO; ++o) mine[o] = out[o];
-    }
-    if (pass == 0) h = v / ((double)mine[1] * nm.sd[1] + nm.mu[1]);
+      for (int o = 0; o < NO; ++o) mine[o] = out[o];
   }
   if (!live) return;
   const double vt = (double)mine[0] * nm.sd[0] + nm.mu[0], vm = (double)mine[2] * nm.sd[2] + nm.mu[2],
