@@ -519,7 +519,7 @@ def run_form(form, nc, fields, cfg, args, diag_steps):
         "roofline": {
             "bound": "hbm",
             "kernel": f"compact line operators along {'xyz'[args.profile_class]} "
-                      f"({'k_line_xu' if args.profile_class == 0 else 'k_line_yz'})",
+                      f"({'k_rhs_x' if args.profile_class == 0 else 'k_rhs_yz'})",
             "achieved": achieved,
             "peak": PEAK_HBM_GBS,
             "unit": "GB/s",
