@@ -443,7 +443,7 @@ __global__ void __launch_bounds__(LPW * A) k_fft2_x_fwd(const T* __restrict__ in
 #pragma unroll
   for (int b = 0; b < B; ++b) {
     const int n = a + A * b;
-    v[b] = cscale(ld_stream(reinterpret_cast<const cx<T>*>(src) + n), in_scale);
+    v[b] = cscale(ld_stream(src + 2 * n), in_scale);
   }
   dft_any<T, B, true>(v);
   twiddle_rows<T, B, true>(v, a, twN);
@@ -534,7 +534,7 @@ __global__ void __launch_bounds__(LPW * A) k_fft2_x_inv(const cx<T>* __restrict_
 #pragma unroll
       for (int k1 = 0; k1 < A; ++k1) {
         const int n = k2 + B * k1;
-        st_stream(reinterpret_cast<cx<T>*>(dst) + n, cscale(u[k1], scale));
+        st_stream(dst + 2 * n, cscale(u[k1], scale));
       }
     }
   }
