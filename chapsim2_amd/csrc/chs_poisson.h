@@ -58,7 +58,7 @@ class Poisson {
   double* yrow = nullptr;                              // y tridiagonal rows: a, c, b, a + c and its rounding (5 ny)
   double *xr = nullptr, *zr = nullptr;                 // eigenvalues of kx (nxh) and kz (nz)
   double* f0 = nullptr;                                // TRID0 factors d, z of the (0, 0) mode (2 ny)
-  double* ya64 = nullptr;                              // longer lines: y lower off-diagonal (ny)
+  double* ya64 = nullptr;                              // longer lines, near-singular modes: y lower off-diagonal (ny)
   double* fd64 = nullptr; double* fz64 = nullptr;      // and per-mode factors (nxh, nz, ny)
   float* fd32 = nullptr; float* fz32 = nullptr;
   void* work = nullptr;                                // complex work (nxh, ny, nz)

@@ -12,7 +12,8 @@
 // nx/2 complex points.
 // The y solves of lines of up to 512 rows are partitioned over the lanes of a
 // workgroup (k_ytdma_part); the mean mode keeps TRID0's order and its
-// singular-pivot rule (|Z| <= 1e-10: last unknown 0) with host-built factors.
+// singular-pivot rule (|Z| <= 1e-10: last unknown 0) with host-built factors,
+// and on domains where other modes come near that rule all modes do.
 #include "chs_poisson.h"
 
 #include <cmath>
@@ -903,7 +904,18 @@ std::string Poisson::create(const Mesh& m, int kind, int iacc, std::unique_ptr<P
   for (int k = 0; k < p->nxh; ++k) mx[k] = mode_root(xrt, p->nx, k);
   for (int k = 0; k < p->nz; ++k) mz[k] = mode_root(zrt, p->nz, k);
   p->td_chunks = (ny + kTdRows - 1) / kTdRows;
-  if (p->td_chunks <= kTdChunks) {
+  // TRID0's rule for a singular last pivot holds for every mode.  The last
+  // pivot grows with the mode's eigenvalue, so the smallest one beside the mean
+  // mode's decides: domains long enough (thousands of channel heights) to bring
+  // it near the rule's 1e-10 keep TRID0's order for all modes.
+  double least = 0.0;
+  for (const std::vector<double>* v : {&mx, &mz})
+    for (double s : *v)
+      if (s < 0.0 && (least == 0.0 || s > least)) least = s;
+  std::vector<double> ld(ny), lz(ny);
+  factors(least, 0.0, ld.data(), lz.data(), 1);
+  const bool near_singular = !(std::fabs(lz[ny - 1]) > 1.0e-6);
+  if (p->td_chunks <= kTdChunks && !near_singular) {
     std::vector<double> row(a), f0(2 * (size_t)ny), sum(ny), low(ny);
     for (int j = 0; j < ny; ++j) {  // a + c = sum + low
       sum[j] = a[j] + c[j];
@@ -915,7 +927,7 @@ std::string Poisson::create(const Mesh& m, int kind, int iacc, std::unique_ptr<P
     if (!(e = upv(row, &p->yrow)).empty() || !(e = upv(f0, &p->f0)).empty()) return e;
     if (!(e = upv(mx, &p->xr)).empty() || !(e = upv(mz, &p->zr)).empty()) return e;
   } else {
-    // lines beyond the partitioned solve: factor tables of every mode
+    // lines beyond the partitioned solve, or near-singular modes: factor tables of every mode
     p->td_chunks = 0;
     if (!(e = upv(a, &p->ya64)).empty()) return e;
     const long nm = (long)p->nxh * p->nz;
