@@ -1151,14 +1151,16 @@ std::string Flow::fused_run(int kind, std::initializer_list<RhsJob<T>> jobs, int
     if (timed) {
       (void)hipEventRecord(e0, s);
       for (int j = 0; j < g.n; ++j) {
-        // fields read and written in T (the second field, the epilogue's), and in FP64
+        // fields read and written in T (the second field, the epilogue's), and in FP64 (the state; a correction's
+        // output, read and written, and the pressure with it)
         const RhsJob<T>& J = g.job[j];
         const double ni = (double)J.nlines * J.p1.n_in, no = (double)J.nlines * J.p1.n_out;
         const double rd[6] = {0, 0, 2, 4, 3, 0}, wr[6] = {1, 2, 1, 3, 1, 0};
         H->prof_bytes += sizeof(T) * (ni * (kind == RK_FINAL ? 2 : 1) + no * (rd[kind] + wr[kind]));
         if (kind == RK_FINAL) H->prof_bytes += J.q ? 16.0 * no : sizeof(T) * no;
         if (kind == RK_FINAL && J.tz == T(0)) H->prof_bytes -= sizeof(T) * no;
-        if (kind == RK_CORRECT) H->prof_bytes += 32.0 * no + (J.out32 ? 4.0 * no : 0.0) + (J.add32 ? 4.0 * no : 0.0);
+        if (kind == RK_CORRECT)
+          H->prof_bytes += no * (16.0 + (J.out32 ? 4.0 : 0.0) + (J.add ? 16.0 : 0.0) + (J.add32 ? 4.0 : 0.0));
       }
     }
     std::string e = dir == 0 ? launch_rhs_x<T>(kind, rows, g, s) : launch_rhs_yz<T>(kind, rows, g, s);
