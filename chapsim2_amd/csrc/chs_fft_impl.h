@@ -547,21 +547,26 @@ __global__ void __launch_bounds__(LPW * A) k_fft2_x_inv(const cx<T>* __restrict_
 // at FP64 took 51 us where the two-pass kernel takes 17 (z lines of 160 on
 // 97 x 96), 19 against 6.3 (x lines of 64, 4096 of them), 45 against 13 (x
 // lines of 192, 15360) and 211 against 58 (z lines of 480, 257 x 64).
-// Lines per workgroup 8 or 16 (v = 0, 1), by timing both once per shape
+// Lines per workgroup 8 or 16 (v = 1, 2), by timing both once per shape
 // (chs_tune.h; 24 against 17 us at 160, 54 against 57 at x lines of 512);
-// untuned shapes use 16 (8 for N = 512).  v = 2, on request only, is the
-// general kernel: it never was the fastest on a length of the list.
+// untuned shapes use 16 (8 for N = 512).  v = 3, on request only, is the
+// general kernel: it never was the fastest on a length of the list.  The
+// numbers stand in saved reports; 0, which was 4 lines per workgroup, takes 8.
 #define CHS_FFT2_LENGTHS(X)                                                                                     \
   X(4, 4) X(4, 5) X(4, 6) X(5, 5) X(3, 9) X(5, 6) X(4, 8) X(6, 6) X(5, 8) X(5, 9) X(6, 8) X(5, 10) X(6, 9)        \
   X(6, 10) X(8, 8) X(8, 9) X(5, 15) X(8, 10) X(9, 9) X(9, 10) X(8, 12) X(10, 10) X(9, 12) X(10, 12) X(8, 16)      \
   X(9, 15) X(12, 12) X(10, 15) X(10, 16) X(9, 18) X(12, 15) X(12, 16) X(10, 20) X(12, 18) X(15, 15) X(15, 16)     \
   X(16, 16) X(15, 18) X(16, 18) X(15, 20) X(16, 20) X(18, 20) X(16, 24) X(20, 20) X(18, 24) X(20, 24) X(16, 32)
-constexpr int kFft2Variants = 2, kFftVariants = 3;
+constexpr int kFft2Variants = 3, kFftVariants = 4;
 
 template <typename T, int A, int B>
 static size_t fft2_lds(int lpw) { return sizeof(cx<T>) * (size_t)lpw * Fft2<A, B>::LSL; }
 
-static int fft2_default_variant(int n) { return n >= 512 ? 0 : 1; }
+// the launch shape of a key: forced or tuned, else by the length
+static int fft2_shape(const std::string& key, int n) {
+  const int v = forced_or_tuned(key, kFftVariants);
+  return v < 0 ? (n >= 512 ? 1 : 2) : v == 0 ? 1 : v;
+}
 
 static std::string fft_key(const char* what, size_t tsize, int n, long nl, long no) {
   return std::string(what) + (tsize == 8 ? "/f64/" : "/f32/") + std::to_string(n) + "/" + std::to_string(nl) + "x" +
@@ -582,8 +587,8 @@ static bool fft2_s_launch(cx<T>* W, int nxh, long ls, int no, long os, const cx<
 template <typename T, int A, int B>
 static bool fft2_s_lpw(int v, cx<T>* W, int nxh, long ls, int no, long os, const cx<T>* tw, T sgn, hipStream_t s) {
   switch (v) {
-    case 0: return fft2_s_launch<T, A, B, 8>(W, nxh, ls, no, os, tw, sgn, s);
-    case 1: return fft2_s_launch<T, A, B, 16>(W, nxh, ls, no, os, tw, sgn, s);
+    case 1: return fft2_s_launch<T, A, B, 8>(W, nxh, ls, no, os, tw, sgn, s);
+    case 2: return fft2_s_launch<T, A, B, 16>(W, nxh, ls, no, os, tw, sgn, s);
   }
   return false;
 }
@@ -616,8 +621,8 @@ template <typename T, int A, int B>
 static bool fft2_x_lpw(int v, bool fwd, const T* in, cx<T>* W, T* out, long nlines, const cx<T>* tw,
                        const cx<T>* rot, T sc, hipStream_t s) {
   switch (v) {
-    case 0: return fft2_x_launch<T, A, B, 8>(fwd, in, W, out, nlines, tw, rot, sc, s);
-    case 1: return fft2_x_launch<T, A, B, 16>(fwd, in, W, out, nlines, tw, rot, sc, s);
+    case 1: return fft2_x_launch<T, A, B, 8>(fwd, in, W, out, nlines, tw, rot, sc, s);
+    case 2: return fft2_x_launch<T, A, B, 16>(fwd, in, W, out, nlines, tw, rot, sc, s);
   }
   return false;
 }
@@ -658,8 +663,7 @@ static void fft_x_general(bool fwd, const T* in, cx<T>* W, T* out, int nx, long 
 template <typename T>
 void launch_fft_s(cx<T>* W, int nxh, int n, long ls, int no, long os, const Radices& rp, const cx<T>* tw,
                          T sgn, hipStream_t s) {
-  int v = forced_or_tuned(fft_key(sgn < T(0) ? "fft_s+" : "fft_s-", sizeof(T), n, nxh, no), kFftVariants);
-  if (v < 0) v = fft2_default_variant(n);
+  const int v = fft2_shape(fft_key(sgn < T(0) ? "fft_s+" : "fft_s-", sizeof(T), n, nxh, no), n);
   if (v < kFft2Variants && fft2_s_variant<T>(v, W, nxh, n, ls, no, os, tw, sgn, s)) return;
   fft_s_general<T>(W, nxh, n, ls, no, os, rp, tw, sgn, s);
 }
@@ -668,8 +672,7 @@ template <typename T>
 void launch_fft_x(bool fwd, const T* in, cx<T>* W, T* out, int nx, long nlines, const Radices& rp,
                          const cx<T>* tw, const cx<T>* rot, T sc, hipStream_t s) {
   const int N = nx / 2;
-  int v = forced_or_tuned(fft_key(fwd ? "fft_x+" : "fft_x-", sizeof(T), N, nlines, 1), kFftVariants);
-  if (v < 0) v = fft2_default_variant(N);
+  const int v = fft2_shape(fft_key(fwd ? "fft_x+" : "fft_x-", sizeof(T), N, nlines, 1), N);
   if (v < kFft2Variants && fft2_x_variant<T>(v, fwd, in, W, out, nx, nlines, tw, rot, sc, s)) return;
   fft_x_general<T>(fwd, in, W, out, nx, nlines, rp, tw, rot, sc, s);
 }
