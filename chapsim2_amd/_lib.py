@@ -22,7 +22,8 @@ EXPORTS = [
     "chs_props_create", "chs_props_destroy", "chs_props_info", "chs_props_from_rhoh", "chs_props_from_h",
     "chs_mlp_create", "chs_mlp_destroy", "chs_mlp_info", "chs_mlp_get_params", "chs_mlp_set_params",
     "chs_mlp_grad", "chs_mlp_train", "chs_mlp_eval",
-    "chs_inspect_coeff", "chs_inspect_op1d", "chs_inspect_projection", "chs_profile_begin", "chs_profile_end", "chs_tune_report",
+    "chs_inspect_coeff", "chs_inspect_op1d", "chs_inspect_projection",
+    "chs_inspect_substep", "chs_profile_begin", "chs_profile_end", "chs_tune_report",
     "chs_op3d_f32", "chs_poisson_f32", "chs_tune_force", "chs_tune_set",
     "chs_props_set_surrogate", "chs_thermo_enable", "chs_thermo_set_rhoh", "chs_thermo_set_mode", "chs_thermo_get",
     "chs_energy_rhs", "chs_mlp_set_matrix_cores",
@@ -126,6 +127,7 @@ def load():
     L.chs_inspect_op1d.argtypes = [C.POINTER(ChsDesc), C.c_int, C.c_int, C.c_int, ip, dp, C.c_int, dp,
                                    C.c_int, dp]
     L.chs_inspect_projection.argtypes = [C.POINTER(ChsDesc), dp, dp, dp, dp, dp]
+    L.chs_inspect_substep.argtypes = [vp, ip]
     L.chs_profile_begin.argtypes = [vp, C.c_int]
     L.chs_profile_end.argtypes = [vp, dp, C.POINTER(C.c_longlong), dp]
     L.chs_tune_report.argtypes = [C.c_char_p, C.c_int]

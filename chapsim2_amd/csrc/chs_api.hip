@@ -738,6 +738,13 @@ int chs_inspect_projection(const chs_desc_t* desc, double* ly, double* lam, doub
 
 extern "C" {
 
+int chs_inspect_substep(chs_handle_t* H, int out[5]) {
+  FLOW_OR_FAIL(H);
+  if (!out) return fail(CHS_EINVAL, "invalid argument");
+  RET(F.substep_path(out));
+  return CHS_OK;
+}
+
 int chs_profile_begin(chs_handle_t* H, int kernel_class) {
   API_CHECK_HANDLE(H);
   if (kernel_class < 0 || kernel_class > 3) return fail(CHS_EINVAL, "kernel class must be 0..3");

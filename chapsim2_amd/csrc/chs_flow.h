@@ -98,6 +98,8 @@ class Flow {
   // also applies the state update (the stored rhs is then only valid for x
   // of a forced flow)
   std::string momentum_rhs(int isub, bool fuse = false);
+  // which operators a sub-step runs (chs_inspect_substep)
+  std::string substep_path(int out[5]);
   std::string divergence(double* div_dev);
   std::string mass_check(double out[3]);
   std::string cfl(double out[2]);   // convective CFL and diffusion numbers
@@ -231,6 +233,7 @@ class Flow {
   FusedPlans<float> f32;
   int rows_yz = 0;            // least chunk length of the fused y and z plans
   int fused_state = 0;        // 0 not decided, 1 fused, 2 single operators
+  bool fuse_short = false;    // the fused plans' chunk form, of every line of the flow
   bool bulk_pending = false;  // qx (gx) holds q + rhs; the forcing's bulk is subtracted by the x correction
   template <typename T> std::string thermo_first_level(RhsWork<T>& w);
   template <typename T> std::string alloc_thermo_work(RhsWork<T>& w);

@@ -1052,15 +1052,14 @@ template <typename T>
 std::string Flow::fused_plans(FusedPlans<T>& f, bool* ok) {
   const int(*B)[5][2] = ibc;
   bool all = true;
-  const bool small = (long)nx * ny * nz <= kShortCells;
   // y and z lines that share launches share the kernel's chunk length
   rows_yz = 0;
   for (auto dn : {std::make_pair(1, ny), std::make_pair(1, py), std::make_pair(2, nz), std::make_pair(2, pz)}) {
     int P, ell, rows;
-    if (fuse_chunks(dn.first, dn.second, small, &P, &ell, &rows)) rows_yz = std::max(rows_yz, rows);
+    if (fuse_chunks(dn.first, dn.second, fuse_short, &P, &ell, &rows)) rows_yz = std::max(rows_yz, rows);
   }
   auto get = [&](const DevFusePlan<T>** p, int dir, int opk, const int* bc, bool fbc, int n_in, int n_out) {
-    std::string e = H->fuse_plan<T>(dir, opk, bc, fbc, n_in, n_out, small, dir ? rows_yz : 0, p);
+    std::string e = H->fuse_plan<T>(dir, opk, bc, fbc, n_in, n_out, fuse_short, dir ? rows_yz : 0, p);
     if (e.empty() && !(*p)->ok) all = false;
     return e;
   };
@@ -1096,14 +1095,31 @@ std::string Flow::fused_ready(bool* ok) {
         same = same && mcov[c][d][0] == BC_PERIODIC && mcov[c][d][1] == BC_PERIODIC;
         for (int v : {VU, VV, VW, VP, VT}) same = same && ibc[d][v][0] == BC_PERIODIC && ibc[d][v][1] == BC_PERIODIC;
       }
-    bool p64 = false, p32 = true;
-    if (same) {
-      SCHK(fused_plans<double>(f64, &p64));
-      if (p64 && mixed) SCHK(fused_plans<float>(f32, &p32));
+    // one chunk form for the whole flow: the short one on small grids where
+    // every line has it (lines of up to 32 chunks), else the long one
+    bool all = false;
+    for (bool shorter : {true, false}) {
+      if (!same || all || (shorter && (long)nx * ny * nz > kShortCells)) continue;
+      fuse_short = shorter;
+      SCHK(fused_plans<double>(f64, &all));
+      if (all && mixed) SCHK(fused_plans<float>(f32, &all));
     }
-    fused_state = same && p64 && p32 ? 1 : 2;
+    fused_state = all ? 1 : 2;
   }
   *ok = fused_state == 1;
+  return "";
+}
+
+std::string Flow::substep_path(int out[5]) {
+  bool fused = false;
+  SCHK(fused_ready(&fused));
+  for (int q = 0; q < 5; ++q) out[q] = 0;
+  if (!fused) return "";
+  out[0] = 1;
+  out[1] = fuse_short;
+  out[2] = f64.xd_c->k.P;
+  out[3] = f64.yd_n->k.P;
+  out[4] = f64.zd_c->k.P;
   return "";
 }
 
@@ -1182,8 +1198,7 @@ template <typename T>
 std::string Flow::plain_job(int dir, int opk, const int* bc, const Field<T>& A, Field<T>& out, const T* fbc, RhsJob<T>* j,
                             bool* ok) {
   const DevFusePlan<T>* p = nullptr;
-  const bool small = (long)nx * ny * nz <= kShortCells;
-  SCHK(H->fuse_plan<T>(dir, opk, bc, fbc != nullptr, A.e.n[dir], out.e.n[dir], small, dir ? rows_yz : 0, &p));
+  SCHK(H->fuse_plan<T>(dir, opk, bc, fbc != nullptr, A.e.n[dir], out.e.n[dir], fuse_short, dir ? rows_yz : 0, &p));
   *ok = p->ok;
   if (!p->ok) return "";
   *j = fused_job<T>(dir, A, out.e, *p);

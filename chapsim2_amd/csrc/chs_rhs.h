@@ -57,9 +57,10 @@ __host__ __device__ constexpr int fuse_band(int rows) {
 // Chunks of a fused plan: P chunks of `ell` rows, the last one shorter (at
 // least two rows); rows, the kernel's chunk length, is 16 or 17, or 8 or 9 in
 // the short form.  x lines take chunks of exactly 16 (8).  y and z lines of a
-// multiple of 16 (8) rows do too, others the fewest chunks of at most 17 (9),
-// so the ny + 1 nodes of a channel with a multiple of 16 cells need no chunk
-// more than its cells.  False beyond kFuseChunks chunks.
+// multiple of 16 (8) rows do too, up to kFuseChunks of them; others take the
+// fewest chunks of at most 17 (9), so the ny + 1 nodes of a channel with a
+// multiple of 16 cells need no chunk more than its cells.  False beyond
+// kFuseChunks chunks.
 // The short form halves each lane's serial work and the code a wave runs
 // through, and doubles the waves: what a small grid wants, whose kernels are
 // bound by both (64^3: see kShortCells in chs_flow.hip).

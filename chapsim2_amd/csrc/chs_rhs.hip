@@ -16,11 +16,11 @@ namespace chs {
 bool fuse_chunks(int dir, int n, bool short_form, int* P, int* ell, int* rows) {
   const int ch = short_form ? 8 : 16;
   if (n < 8) return false;
-  if (dir == 0 || n % ch == 0) {
-    const int p = (n + ch - 1) / ch;
-    *P = p;
+  const int whole = (n + ch - 1) / ch;
+  if (dir == 0 || (n % ch == 0 && whole <= kFuseChunks)) {
+    *P = whole;
     *ell = *rows = ch;
-    return p <= kFuseChunks && n - ch * (p - 1) >= 2;
+    return whole <= kFuseChunks && n - ch * (whole - 1) >= 2;
   }
   for (int p = (n + ch) / (ch + 1); p <= kFuseChunks; ++p) {
     const int l = (n + p - 1) / p;

@@ -35,6 +35,13 @@ int chs_inspect_op1d(const chs_desc_t *desc, int dir, int op, int iacc, const in
 int chs_inspect_projection(const chs_desc_t *desc, double *ly, double *lam, double *lx, double *lz,
                            double *resid);
 
+/* Which line operators the handle's sub-steps run (decided on the GPU the
+ * first time a sub-step or this call needs it): out[0] 1 for the fused ones,
+ * 0 for one operator per launch; with 1, out[1] 1 for chunks of at most 9 rows
+ * and 0 for chunks of at most 17, and out[2..4] the chunks of an x line, of a
+ * y line of nodes and of a z line (0 otherwise). */
+int chs_inspect_substep(chs_handle_t *h, int out[5]);
+
 /* Launch timing of one kernel class during subsequent solver and chs_op3d
  * calls, with HIP events on the handle's stream: class 0/1/2 = x/y/z line
  * operators, 3 = whole chs_poisson / chs_poisson_f32 solves (counted as five
