@@ -511,11 +511,14 @@ static std::string batch_capture(chs_batch* b) {
     if (hipStreamWaitEvent(h.stream, b->fork, 0) != hipSuccess) { err = "fork wait"; break; }
     // the captured step starts from fresh FP32 copies of the state (a replay
     // follows a step, which leaves them so, or chs_batch_run's rounding of
-    // an instance whose state was set); the flag is restored after capture
-    const bool fresh = h.flow->q32_fresh;
+    // an instance whose state was set); capturing runs nothing, so the flags
+    // of the FP32 copies are restored after it
+    const bool q32 = h.flow->q32_fresh, g32 = h.flow->g32_fresh, props32 = h.flow->props32_fresh;
     h.flow->q32_fresh = true;
     for (int isub = 1; isub <= 3 && err.empty(); ++isub) err = h.flow->substep(isub);
-    h.flow->q32_fresh = fresh;
+    h.flow->q32_fresh = q32;
+    h.flow->g32_fresh = g32;
+    h.flow->props32_fresh = props32;
     if (err.empty() && hipEventRecord(b->join[i], h.stream) != hipSuccess) err = "join record";
     if (err.empty() && hipStreamWaitEvent(b->main, b->join[i], 0) != hipSuccess) err = "join wait";
   }
