@@ -224,7 +224,7 @@ class Flow {
   template <typename T> std::string wall_stress(RhsWork<T>& w, const T* conv);
   template <typename T> std::string fused_plans(FusedPlans<T>& f, bool* ok);
   template <typename T>
-  std::string fused_run(int kind, std::initializer_list<RhsJob<T>> jobs, int lane = 0);
+  std::string fused_run(int kind, std::initializer_list<RhsJob<T>> jobs);
   std::string fused_ready(bool* ok);  // every operator of the sub-step has its fused plan (decided once)
   std::string divergence_fused(double* d);
   std::string correct(double sc);  // p += phi and the velocity correction

@@ -718,7 +718,7 @@ std::string Flow::op(RhsWork<T>& w, int dir, int opk, const int ibc2[2], const F
     RhsJob<T> j{};
     bool ok = false;
     SCHK(plain_job<T>(dir, opk, ibc2, A, out, fbc, &j, &ok));
-    if (ok) return fused_run<T>(RK_SINGLE, {j}, lane);
+    if (ok) return fused_run<T>(RK_SINGLE, {j});
   }
   const DevPlan<T>* P = nullptr;
   SCHK(H->plan<T>(dir, opk, H->desc.iacc, ibc2, fbc != nullptr, A.e.n[dir], out.e.n[dir], &P));
@@ -1152,8 +1152,8 @@ static RhsJob<T> fused_job(int dir, const Field<T>& A, const Ext3& eo, const Dev
 }
 
 template <typename T>
-std::string Flow::fused_run(int kind, std::initializer_list<RhsJob<T>> jobs, int lane) {
-  const hipStream_t s = lane_stream(lane);
+std::string Flow::fused_run(int kind, std::initializer_list<RhsJob<T>> jobs) {
+  const hipStream_t s = H->stream;  // (no side streams on this path: set_lanes)
   // (launch profiling times each operator; otherwise jobs of one kind share a
   // launch on any grid: two RK3 steps of 192x96x160 FP64 4.42 -> 4.17 ms, of
   // 128x96x128 mixed 2.40 -> 2.00, of 256x128x256 9.95 -> 9.79)
