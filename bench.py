@@ -442,7 +442,7 @@ def batch_bench(args):
 
 FORMS = {
     "fp64c": "FP64 throughout, exact projection (inverse of the compact D*G per sub-step)",
-    "mixed": "FP32 momentum right-hand side (44 line operators, products, fractional step); FP64 state, "
+    "mixed": "FP32 momentum right-hand side (30 line operators with the fluxes and the fractional step in them); FP64 state, "
              "bulk-flux sums, divergence, exact projection and correction",
     "fp64r": "FP64 with the reference's single FFT(x,z)+TDMA(y) 2nd-order projection per sub-step",
 }

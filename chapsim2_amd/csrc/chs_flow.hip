@@ -1045,8 +1045,12 @@ std::string Flow::momentum_rhs_t(RhsWork<T>& w, int isub, bool fuse) {
 // ---------------------------------------------------------------------------
 // The sub-step on the fused operators (chs_rhs.h)
 // ---------------------------------------------------------------------------
-// Grids of up to this many cells take the short chunks (beyond, the long ones
-// are faster: two RK3 steps of 160x96x128 FP64 2.97 ms against 3.29).
+// Grids of up to this many cells take the short chunks.  Sub-steps with the
+// short and the long ones, us, FP64 and mixed: 64^3 176, 153 and 203, 175;
+// 96x64x64 200, 163 and 219, 184; 96x96x64 229, 184 and 245, 203; 128x64x96 277,
+// 211 and 273, 219; 128x96x96 345, 250 and 334, 255; 128^3 523, 363 and 463,
+// 352.  They meet at 0.8 million cells in FP64 and at 1.3 in the mixed form; the
+// line stays below both.
 constexpr long kShortCells = 1L << 19;
 template <typename T>
 std::string Flow::fused_plans(FusedPlans<T>& f, bool* ok) {

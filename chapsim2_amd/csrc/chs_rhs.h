@@ -20,13 +20,15 @@
 // together, which is what small grids need: their launches are latency (ten
 // RK3 steps of 64^3 with y and z apart and the corrections on side streams
 // 7.06 ms, now 4.6).
-// Two RK3 steps at 256x128x256 with the state's copies in and out: FP64 12.86
-// -> 9.95 ms, mixed 9.21 -> 7.35 ms; three of six uneven channels as one graph
-// 15.5 -> 10.4 ms; ten of 64^3 9.7 -> 4.6 ms.  What bounds the large grids is
+// Two RK3 steps at 256x128x256 with the state's copies in and out: FP64 12.8
+// -> 9.8 ms, mixed 9.2 -> 7.2 ms; three of six uneven channels as one graph
+// 15.5 -> 10.2 ms; ten of 64^3 9.0 -> 4.6 ms.  What bounds the large grids is
 // memory: the fields moved per sub-step (about 102 with the projection, 139
-// before) at the rate of a large copy (4.8 TB/s); the small ones are bound by
-// each launch's serial chain (arguments, one round trip to memory, the solve,
-// the stores) and by the code a wave fetches once.
+// before) at up to the rate of a large copy (4.8 TB/s); in FP64 the register
+// spills of the last x operator (132 bytes per lane) and of the normal fluxes
+// add 29 and 13 % to those kernels' bytes.  The small grids are bound by each
+// launch's serial chain (arguments, one round trip to memory, the solve, the
+// stores) and by the code a wave fetches once.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -47,8 +49,12 @@ enum FuseCo : int { FC_LD = 0, FC_AL = 1, FC_SV = 2, FC_SW = 3, FC_LC = 4 };
 // inverse of the reduced system falls off per row with the scheme's decay rate
 // (at most 1/3), so the ends of the next d chunks on either side (4 d + 4
 // values) hold every term above 2^-59 (FP64) or 2^-36 (FP32) of the largest:
-// d = 2 and 1 for chunks of 13 rows and more, 4 and 2 for shorter ones (checked
-// against the whole inverse when the plan is made).
+// d = 2 and 1 for the kernels of 16 and 17 rows, 4 and 2 for those of 8 and 9.
+// That is checked against the whole inverse when the plan is made.  A short
+// last chunk brings the ends beyond it nearer, so a periodic line of many chunks
+// whose last has some 2 to 4 rows is refused (x lines of 100, 162, 180, 324, 450
+// and 500, in FP32 also 150 and 486; z lines of 324 and 360; in the short form
+// more of them) and its flow runs single operators.
 template <typename T>
 __host__ __device__ constexpr int fuse_band(int rows) {
   return rows >= 16 ? (sizeof(T) == 8 ? 12 : 8) : (sizeof(T) == 8 ? 20 : 12);
@@ -63,7 +69,7 @@ __host__ __device__ constexpr int fuse_band(int rows) {
 // kFuseChunks chunks.
 // The short form halves each lane's serial work and the code a wave runs
 // through, and doubles the waves: what a small grid wants, whose kernels are
-// bound by both (64^3: see kShortCells in chs_flow.hip).
+// bound by both (kShortCells in chs_flow.hip has the figures).
 bool fuse_chunks(int dir, int n, bool short_form, int* P, int* ell, int* rows);
 
 // Kernel view of a fused plan: a staggered operator (interpolation or first
@@ -143,7 +149,8 @@ struct RhsGroup {
 // (periodic, contiguous, n_in = n_out), or y and z lines in any mixture.
 template <typename T>
 std::string launch_rhs_x(int kind, int rows, RhsGroup<T>& g, hipStream_t s);
-// y and z lines; the jobs' plans have the same number of chunks.
+// y and z lines: the workgroups have lanes for the most chunks of a job (G.P); a
+// job's plans have one geometry, and all tables are laid out for `rows`.
 template <typename T>
 std::string launch_rhs_yz(int kind, int rows, RhsGroup<T>& g, hipStream_t s);
 // number of blocks launch_rhs_x takes for one job (entries of its partial sums)

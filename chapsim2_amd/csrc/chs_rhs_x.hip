@@ -294,7 +294,10 @@ __global__ void __launch_bounds__(64 * kXWaves) __attribute__((amdgpu_waves_per_
 }
 
 // Waves per workgroup: as many as share the tables, but no fewer workgroups
-// than the CUs have room for (64 x 64 lines of 64 points are 256 waves).
+// than the CUs have room for.  FP64 sub-steps with 1, 2 and 4 waves: 64^3 (512
+// waves of x lines) 177, 175, 174 us, 128x96x96 (1152) 344, 335, 341, 192x96x160
+// (3072) 705, 676, 675, 256x128x256 (8192) 1685, 1642, 1589; below 1024 waves
+// the choice is worth 2 % at most.
 static int x_waves(long waves) { return waves >= 2048 ? kXWaves : waves >= 1024 ? 2 : 1; }
 
 template <typename T>

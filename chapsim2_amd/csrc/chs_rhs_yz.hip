@@ -289,13 +289,18 @@ std::string launch_rhs_yz(int kind, int rows, RhsGroup<T>& G, hipStream_t s) {
   for (int j = 0; j < G.n; ++j) P = std::max(P, G.job[j].p1.P);
   if (P < 1 || P > kFuseChunks) return "fused yz: bad chunks";
   G.P = P;
+  // 64 lines per workgroup up to 16 chunks of 8 or 9 rows (8 of 16 or 17): at
+  // 256x128x256, where only lines of up to 8 chunks take them, a sub-step is as
+  // fast with 32 lines throughout (1591 us FP64, 1124 mixed) and slower with 64
+  // for 16 chunks too (1609, 1148).  On small grids the two are within 3 %: 129 us
+  // against 132 at 32x24x16, 177 against 172 at 64^3, 200 against 195 at 96x64x64.
   const bool wide = rows < 16 ? P <= 16 : P <= 8;
   const int nlw = wide ? 64 : 32;
   size_t tab = 0;
   G.first[0] = 0;
   for (int j = 0; j < G.n; ++j) {
     const RhsJob<T>& J = G.job[j];
-    if (J.p1.P < 1 || J.rows != rows || J.p1.ell > rows) return "fused yz: the group's plans differ in chunks";
+    if (J.p1.P < 1 || J.rows != rows || J.p1.ell > rows) return "fused yz: a plan of another chunk length";
     if (two && (J.p2.P != J.p1.P || J.p2.ell != J.p1.ell || J.p2.n_in != J.p1.n_in || J.p2.n_out != J.p1.n_out ||
                               J.p2.sh != J.p1.sh || J.p2.wrap != J.p1.wrap))
       return "fused yz: a job's two plans differ in geometry";
