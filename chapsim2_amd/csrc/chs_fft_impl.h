@@ -542,7 +542,7 @@ __global__ void __launch_bounds__(LPW * A) k_fft2_x_inv(const cx<T>* __restrict_
 
 // Launchers: the two-pass kernels for the lengths below (all 2,3,5-smooth ones
 // from 16 to 512 but 18, 125, 243, 250, 324, 375, 405, 450, 486 and 500, which
-// no case has and nobody timed in two passes), the general Stockham kernels
+// were not timed in two passes), the general Stockham kernels
 // otherwise: those pass every element through LDS once per prime factor, and
 // at FP64 took 51 us where the two-pass kernel takes 17 (z lines of 160 on
 // 97 x 96), 19 against 6.3 (x lines of 64, 4096 of them), 45 against 13 (x

@@ -46,8 +46,8 @@ int chs_inspect_substep(chs_handle_t *h, int out[5]);
  * calls, with HIP events on the handle's stream: class 0/1/2 = x/y/z line
  * operators, 3 = whole chs_poisson / chs_poisson_f32 solves (counted as five
  * passes that each read and write the field).  While a class is profiled,
- * sub-steps issue every kernel on the handle's stream, one at a time (they
- * otherwise overlap independent operators on side streams), so each timed
+ * sub-steps issue every operator on the handle's stream, one at a time (they
+ * otherwise share launches or overlap on side streams), so each timed
  * launch has the GPU to itself.  chs_profile_end returns the summed
  * event time, the number of timed launches and their algorithmic bytes
  * (arrays read plus arrays written, 8 bytes per FP64 and 4 per FP32
@@ -64,7 +64,8 @@ int chs_op3d_f32(chs_handle_t *h, int dir, int op, int iacc, const int ibc[2], c
                  const int shp_in[3], float *fo, const int shp_out[3], const float *fbc);
 int chs_poisson_f32(chs_handle_t *h, float *rhs);
 
-/* Launch shapes chosen so far by the autotuner (FFT lines per workgroup,
+/* Launch shapes chosen so far by the autotuner (FFT lines per workgroup: 1 for 8,
+ * 2 for 16, 3 the general kernel;
  * x-line tile), one "family/shape=choice (us per variant)" line each, for
  * every handle of the process.  Writes at most len-1 characters and a
  * terminating 0; returns the number of tuned shapes.  No counterpart in the
